@@ -65,16 +65,6 @@ __device__ __forceinline__ void store_block9(double *dst, const double (&b)[9])
     dst[8] = b[8];
 }
 
-// lap stage slot: vertex v's gradient {x, y, z}.
-template <typename T, typename T2>
-__device__ __forceinline__ void stage_grad(const T *sl, int v, T (&g)[3])
-{
-    const T2 xy = *reinterpret_cast<const T2 *>(sl + 2 * v);
-    g[0] = xy.x;
-    g[1] = xy.y;
-    g[2] = sl[8 + v];
-}
-
 // ela stage slot: vertex v's group {gx, gy, gz, lambda+2mu} at sl + 4v (16-byte aligned).
 __device__ __forceinline__ void ela_vertex(const double *p, double (&g)[3], double &cd)
 {
@@ -272,13 +262,19 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
             for (int i = 0; i < 4; i++) ela_vertex_store(sl + 4 * i, g[i], cd);
             *reinterpret_cast<T2 *>(sl + 16) = T2{(T)co, (T)cm};
         } else {
+            // the element matrix, each product as the block sums take it
+            const T kk = (T)reinterpret_cast<const double *>(lds_raw + L.coef)[t];
+            T gt[4][3], m[10];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                *reinterpret_cast<T2 *>(sl + 2 * i) = T2{(T)g[i][0], (T)g[i][1]};
-                sl[8 + i] = (T)g[i][2];
-            }
-            const double kk = reinterpret_cast<const double *>(lds_raw + L.coef)[t];
-            *reinterpret_cast<T2 *>(sl + 12) = T2{(T)kk, (T)0};
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int d = 0; d < 3; d++) gt[i][d] = (T)g[i][d];
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = i; j < 4; j++) m[mf::lap_slot(i, j)] = kk * mf::lap_entry(gt[i], gt[j]);
+#pragma unroll
+            for (int q = 0; q < 10; q += 2) *reinterpret_cast<T2 *>(sl + q) = T2{m[q], m[q + 1]};
         }
     }
     // the zero slot (index TE): the target of an unpaired second contribution
@@ -323,7 +319,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
         auto word = [&](int q) { return lw[q < lastw ? q : lastw]; };
         struct Pair {
             T g[2][3];
-            T c[2][3];  // ela: lambda + 2 mu, lambda + mu, mu; lap: k
+            T c[2][3];  // ela: lambda + 2 mu, lambda + mu, mu; lap: the product itself
         };
         auto fetch = [&](uint32_t w, Pair &P) {
 #pragma unroll
@@ -336,8 +332,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
                     P.c[u][1] = c12.x;
                     P.c[u][2] = c12.y;
                 } else {
-                    stage_grad<T, T2>(sl, e & 3, P.g[u]);
-                    P.c[u][0] = sl[12];
+                    P.c[u][0] = sl[e & 3];
                 }
             }
         };
@@ -348,8 +343,8 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 if (2 * p + u >= val) break;
-                const T *g = P.g[u];
                 if constexpr (ELA) {
+                    const T *g = P.g[u];
                     const T cd = P.c[u][0], co = P.c[u][1], cm = P.c[u][2];
                     const T p00 = g[0] * g[0], p11 = g[1] * g[1], p22 = g[2] * g[2];
                     s0 += (double)(p00 * cd + p11 * cm + p22 * cm);
@@ -359,8 +354,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
                     s5 += (double)(g[1] * g[2] * co);
                     s8 += (double)(p00 * cm + p11 * cm + p22 * cd);
                 } else {
-                    const T x = P.c[u][0] * mf::lap_entry(g, g);
-                    s0 += (double)x;
+                    s0 += (double)P.c[u][0];
                 }
             }
         };
@@ -416,9 +410,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
                     c1[u] = c12.x;
                     c2[u] = c12.y;
                 } else {
-                    stage_grad<T, T2>(sl, a[u], ga[u]);
-                    stage_grad<T, T2>(sl, kk[u], gk[u]);
-                    c0[u] = sl[12];
+                    c0[u] = sl[mf::lap_slot(a[u], kk[u])];
                 }
             }
 #pragma unroll
@@ -429,8 +421,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
 #pragma unroll
                     for (int q = 0; q < 9; q++) acc[q] += (double)bl[q];
                 } else {
-                    const T x = c0[u] * mf::lap_entry(ga[u], gk[u]);
-                    acc[0] += (double)x;
+                    acc[0] += (double)c0[u];
                 }
             }
         };
