@@ -212,10 +212,13 @@ int mf_hbm_copy(void *dst, const void *src, size_t bytes, void *stream);
 int mf_gather_probe(double *dst, const double *src, const int64_t *idx, int64_t n, void *stream);
 
 /* assembly (src/headers/assembly.h:61-74, called at src/FEM.cc:183), COLORING
- * semantics (src/assembly.cc:593-611, :660-673): zero values[nbEdges*operatorDim],
- * then one race-free launch per color over elements [colorToElem[c], colorToElem[c+1])
- * of the color-permuted elemToNode. elemToEdge (device, 16 per element) gives the
- * scatter positions; NULL selects the reference's default row search
+ * semantics (src/assembly.cc:593-611, :660-673): values[nbEdges*operatorDim] receive, each
+ * entry from zero and in color order, the blocks of elements [colorToElem[c],
+ * colorToElem[c+1]), c = 0, 1, ..., of the color-permuted elemToNode (elements of one color
+ * share no node). The call takes stream-ordered workspace from a pool of the library's own,
+ * about 1 byte per CSR entry and color (4 with elemToEdge); under stream capture, or where
+ * there is no memory for it, it runs one launch per color instead. elemToEdge (device, 16
+ * per element) gives the scatter positions; NULL selects the reference's default row search
  * (src/assembly.cc:415-421). colorToElem is a HOST array of nbColors+1 offsets (the
  * reference's global). Device: coord, values, row, col, elemToNode, elemToEdge. */
 int mf_assembly(const double *coord, double *values, const int *row, const int *col,
