@@ -194,15 +194,6 @@ __global__ void __launch_bounds__(1024)
 // ela 60^3 1,830 -> 416 us, lap 31^3 with elemToEdge 148 -> 53 (the two prec
 // calls included); ela 60^3: k_row_table 63 us, k_assemble_rows 293.
 
-// Orders a wave's LDS accesses: LDS operations of one wave complete in order, so only the
-// compiler has to be told.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The color of element e, one of the n from e0 (the same for the whole wave) on: e0's by
 // bisection, then the few that the n span.
 __device__ __forceinline__ int color_of(const ColorOffsets &co, int e0, int e, int n)
@@ -339,7 +330,7 @@ __global__ void __launch_bounds__(64)
         }
         const int len = r1 - r0;
         const int key0 = EDGES ? r0 + l : l < len ? col[r0 + l] : 0;
-        wave_sync();  // the previous rows' reads
+        mf::wave_sync();  // the previous rows' reads
         int L = 0;
 #pragma unroll
         for (int k = 0; k < KC; k++) {
@@ -381,7 +372,7 @@ __global__ void __launch_bounds__(64)
                 for (int ch = 0; ch < nch; ch++) {
                     const int Lc = L - ch * SL < SL ? L - ch * SL : SL;
                     if (nch > 1 || pass == 0) {
-                        wave_sync();  // the list is written, the previous chunk read
+                        mf::wave_sync();  // the list is written, the previous chunk read
                         // the loads of both of a lane's elements go out together
                         double c[H][4][3], kl[H];
                         mf::ElaCoef kc[H];
@@ -449,7 +440,7 @@ __global__ void __launch_bounds__(64)
                                 }
                             }
                         }
-                        wave_sync();
+                        mf::wave_sync();
                     }
                     // bit s of m[k]: the chunk's s-th element holds this entry as its vertex k
                     uint32_t m[4] = {0, 0, 0, 0};
@@ -515,7 +506,7 @@ __global__ void __launch_bounds__(64)
                     // the stage is needed for nothing else in this chunk: the diagonal values
                     // of its elements go over their gradients
                     if (nch > 1 ? pass == 0 : pass == npass - 1) {
-                        wave_sync();
+                        mf::wave_sync();
                         if constexpr (ELA) {
 #pragma unroll
                             for (int h = 0; h < H; h++) {
@@ -531,7 +522,7 @@ __global__ void __launch_bounds__(64)
                                 o[4] = y * z * c1;
                                 o[5] = p00 * cm + p11 * cm + p22 * cd;
                             }
-                            wave_sync();
+                            mf::wave_sync();
                         }
                         if (l < (ELA ? 6 : 1)) {
                             for (int q = 0; q < Lc; q += 4) {
@@ -542,7 +533,7 @@ __global__ void __launch_bounds__(64)
                                 for (int u = 0; u < 4; u++) dsum += (double)x[u];
                             }
                         }
-                        wave_sync();
+                        mf::wave_sync();
                     }
                 }
                 if (p < r1 && dpos != p) {
@@ -569,12 +560,12 @@ __global__ void __launch_bounds__(64)
             // a vertex matched by two entries: a column stands twice in the row
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) matched += __shfl_xor(matched, o, 16);
-            wave_sync();
+            mf::wave_sync();
             int seen = 0;
             for (int q = l; q < CH * 4; q += 16) seen += __builtin_popcount(s_seen[g][q]);
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) seen += __shfl_xor(seen, o, 16);
-            wave_sync();
+            mf::wave_sync();
             if (!__ballot(matched != seen)) break;
         }
         r0 = r0n;
@@ -761,37 +752,6 @@ int launch_colors(const double *coord, const double *coef, double *values, const
     return MF_OK;
 }
 
-// The device's own pool of stream-ordered memory for the workspaces of calls that do not
-// wait for their work: it keeps up to kPoolKeep bytes between calls (the default pool gives
-// everything back at each synchronization, and taking 100 MB again costs 0.3 ms), and
-// hipFreeAsync makes it safe for several streams and threads.
-constexpr uint64_t kPoolKeep = 512ull << 20;
-std::mutex g_pool_mu;
-hipMemPool_t g_pool[64] = {};
-
-hipMemPool_t workspace_pool()
-{
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-    std::lock_guard<std::mutex> lock(g_pool_mu);
-    if (!g_pool[dev]) {
-        hipMemPoolProps props{};
-        props.allocType = hipMemAllocationTypePinned;
-        props.location.type = hipMemLocationTypeDevice;
-        props.location.id = dev;
-        hipMemPool_t pool = nullptr;
-        uint64_t keep = kPoolKeep;
-        if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
-        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
-            (void)hipMemPoolDestroy(pool);
-            return nullptr;
-        }
-        g_pool[dev] = pool;
-    }
-    return g_pool[dev];
-}
-
-
 template <int OP, int PREC, bool EDGES>
 void launch_rows_width(int kc, const ColorOffsets &co, const double *coord, const double *coef,
                        double *values, const int *row, const int *col, const int4 *e2n,
@@ -826,7 +786,7 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
         (void)hipGetLastError();
         return false;
     }
-    hipMemPool_t pool = workspace_pool();
+    hipMemPool_t pool = mf::workspace_pool();
     if (!pool) return false;
     ColorOffsets co;
     co.n = nbColors;
@@ -956,7 +916,7 @@ extern "C" int mf_device_init(int device)
                      device, prop.gcnArchName);
         return MF_ERR_HIP;
     }
-    (void)workspace_pool();  // made here rather than in a call's first use
+    (void)mf::workspace_pool();  // made here rather than in a call's first use
     double *unused = nullptr;
     return norm_scratch(device, &unused);
 }

@@ -16,6 +16,54 @@
 
 namespace mf {
 
+// Orders a wave's LDS accesses: LDS operations of one wave complete in order, so only the
+// compiler has to be told.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The current device's own pool of stream-ordered memory, for the workspaces of calls
+// (device_runtime.hip); null when it cannot be made. hipFreeAsync makes it safe for several
+// streams and threads.
+hipMemPool_t workspace_pool();
+
+// One block of workspace, taken from the pool on construction and given back, in stream
+// order, on destruction. Pieces are cut from it in turn, 256-byte aligned.
+class Workspace {
+public:
+    Workspace(size_t bytes, hipStream_t s) : s_(s), size_(bytes)
+    {
+        hipMemPool_t pool = workspace_pool();
+        if (!pool || hipMallocFromPoolAsync(reinterpret_cast<void **>(&base_), bytes, pool, s) != hipSuccess) {
+            (void)hipGetLastError();
+            base_ = nullptr;
+        }
+    }
+    ~Workspace()
+    {
+        if (base_) (void)hipFreeAsync(base_, s_);
+    }
+    Workspace(const Workspace &) = delete;
+    Workspace &operator=(const Workspace &) = delete;
+    bool ok() const { return base_ != nullptr; }
+    static size_t padded(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    template <typename T>
+    T *cut(size_t n)
+    {
+        T *p = reinterpret_cast<T *>(base_ + used_);
+        used_ += padded(n * sizeof(T));
+        return used_ <= size_ ? p : nullptr;
+    }
+
+private:
+    hipStream_t s_;
+    unsigned char *base_ = nullptr;
+    size_t size_, used_ = 0;
+};
+
 // Scaled P1 gradients of one tet, src/assembly.cc:85-121: a=v0-v3, b=v2-v3, c=v1-v3,
 // g0=b x c, g1=a x b, g2=c x a, g3=-(g0+g1+g2), det=a.g0, g *= (1./det).
 __device__ __forceinline__ void elem_grad(const double (&c)[4][3], double (&g)[4][3])

@@ -136,3 +136,39 @@ def test_mesh_device_setup_equals_host(mf, gpu, n, op, shuffle):
     for name in ("elemToNode", "coef", "colorPerm", "colorToElem", "row", "col", "checkBounds"):
         assert np.array_equal(getattr(h, name), getattr(d, name)), name
     assert h.nnz == d.nnz
+
+
+def _tets(rng, nodes, n, repeat=0.0):
+    """n tets of random nodes; a share of them with a vertex twice."""
+    t = np.stack([rng.permutation(nodes)[:4] for _ in range(n)]) + 1
+    twice = rng.random(n) < repeat
+    t[twice, 3] = t[twice, rng.integers(0, 3, twice.sum())]
+    return t.astype(np.int32).ravel()
+
+
+@pytest.mark.parametrize("what", ["one", "sparse", "repeats", "dense", "fan40", "fan41", "fan90"])
+def test_chains_and_rows_equal_host(mf, gpu, what):
+    """Coloring by chains and by levels, and rows of up to and past 64 elements."""
+    rng = np.random.default_rng(8)
+    if what.startswith("fan"):  # so many tets around one edge: 40 is the chains' last valence
+        n = int(what[3:])
+        e2n, N = np.array([[1, 2, 3 + k, 3 + (k + 1) % n] for k in range(n)], np.int32), n + 2
+        e2n = rng.permutation(e2n).ravel()
+    else:
+        N, nE, rep = {"one": (4, 1, 0), "sparse": (3000, 9000, 0), "repeats": (500, 1500, 0.3),
+                      "dense": (1200, 6000, 0.05)}[what]
+        e2n = _tets(rng, N, nE, rep)
+    print(f"[setup chains] {what}", flush=True)
+    part, perm, c2e = gpu.coloring_creation(e2n, N)
+    hp, hperm, hc2e = mf.coloring_creation(e2n, N)
+    assert np.array_equal(part.numpy(), hp) and np.array_equal(perm.numpy(), hperm)
+    assert np.array_equal(c2e, hc2e)
+    index, value = mf.create_nodeToElem(e2n, N)
+    cap = 16 * (e2n.size // 4) + N
+    row, col = mf.create_nodeToNode(e2n, N, cap)
+    d = gpu.device_setup(e2n, N, cap)
+    assert d[5] == row[-1]
+    assert np.array_equal(d[0].numpy(), index) and np.array_equal(d[1].numpy(), value[:e2n.size])
+    assert np.array_equal(d[2].numpy(), row)
+    assert np.array_equal(d[3].numpy()[:d[5]], col[:d[5]])
+    assert np.array_equal(d[4].numpy(), mf.create_elemToEdge(row, col, e2n))
