@@ -45,8 +45,9 @@ __global__ void __launch_bounds__(256)
 namespace mf {
 
 // It keeps up to kPoolKeep bytes between calls: the default pool gives everything back at each
-// synchronization, and taking 100 MB again costs 0.3 ms.
-constexpr uint64_t kPoolKeep = 512ull << 20;
+// synchronization, and taking 100 MB or more again costs 0.3 ms (with 2 GiB: the workspace of a
+// solve or of a drop-in call with elemToEdge at a million nodes; 0.7 % of the HBM).
+constexpr uint64_t kPoolKeep = 2ull << 30;
 
 hipMemPool_t workspace_pool()
 {

@@ -10,25 +10,30 @@
 // so z = prec r is the block-Jacobi step. Diagonal blocks of ela are symmetric, so the
 // Fortran column-major and C row-major views of prec coincide.
 //
-// One iteration is three streaming launches, each reading what it needs once, and two
-// one-workgroup sums of their partials; the scalars stay on the device:
-//   q = K p with the partial sums of p.q          (k_spmv, k_spmv_ela_staged: 16 lanes
-//                                                   per row; k_sum_pq)
+// One iteration is three launches, each reading what it needs once; the scalars stay on the
+// device:
+//   q = K p with the partial sums of p.q           (k_spmv_lap, k_spmv_ela_staged:
+//                                                   16 lanes per row)
 //   x += alpha p, r -= alpha q, z = M r with the partial sums of r.z and r.r
-//                                                  (k_update_prec_dot; k_sum_rz)
-//   p = z + beta p and its masked copy P p         (k_xpby)
+//                                                  (k_update_prec_dot)
+//   p = z + beta p and its masked copy P p, and the next iteration's scalars  (k_direction)
+// Every workgroup of the second and third sums the launch before's partials for itself, in
+// one fixed order, instead of waiting for a launch that sums them: 2,048 partials are 16 KB
+// of L2 reads each, less than the start of a launch (an iteration of lap 41^3 27 -> 22 us, of
+// ela 80^3 in the plan's order 185 -> 176, 100^3 351 -> 320).
 // The product reads each row's blocks as one contiguous stream: the 16 lanes of a row
 // take its blocks in turn (consecutive lanes, consecutive 72- or 8-byte blocks), then
 // sum their three (one) partial rows in a fixed butterfly; the columns are gathered
 // from the masked copy of the direction, one gather per block. Dot products are
 // deterministic: a fixed grid, a fixed tree per workgroup, the workgroup partials summed
-// in a fixed tree by one workgroup, and only that scalar goes to the host.
+// in a fixed tree.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <type_traits>
 
 #include "device_common.h"
 #include "minifem.h"
@@ -36,18 +41,18 @@
 namespace {
 
 constexpr int kBT = 256;          // threads per workgroup
-constexpr int kGroup = 16;        // lanes per row in the operator product (ela)
-// lanes per row of the lap product: 8 took 82 against 87 us per lap 100^3 iteration in the
-// plan's order but 217 against 204 us in the shuffled one, 4 was slower in both
-constexpr int kLapGroup = 16;
+// lanes per row in the operator product; for lap 8 took 82 against 87 us per 100^3 iteration
+// in the plan's order but 217 against 204 us in the shuffled one, 4 was slower in both
+constexpr int kGroup = 16;
 constexpr int kMaxGrid = 2048;    // workgroups of the reducing kernels (partials per sum)
 constexpr int kBatch = 8;         // iterations enqueued between two looks at the state
 
 // The iteration's scalars, on the device: the host enqueues iterations without waiting
-// for them and reads this every kBatch iterations. Once done is set, every kernel of
-// the iterations already enqueued returns at once.
+// for them and reads this after every kBatch. There are two: an iteration reads one and
+// k_direction writes the other, so no workgroup reads what another one writes. Once done is
+// set, every kernel of the iterations already enqueued returns at once.
 struct CgState {
-    double rz, rz1, rr, pq, beta, tol;
+    double rz, rr, tol, bnorm;
     int it, max_it;
     int done;  // 0 running; 1 converged or max_it reached; 2 p.q <= 0 (breakdown)
     int pad;
@@ -69,81 +74,89 @@ __global__ void k_mask_bits(const int *__restrict__ cb, int N, bool ela, const i
     m[t] = b;
 }
 
-// Fixed-order sum of the kBT values of a workgroup in s[]; returns it on thread 0.
-__device__ __forceinline__ double block_sum(double *s, double v)
+// Sum of x over the 16 lanes of a row, on every one of them (cross-lane moves of the vector
+// unit, which leave the LDS to the operands).
+__device__ __forceinline__ double row16_sum(double x)
 {
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = kBT / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    const double r = s[0];
-    __syncthreads();
-    return r;
+    auto moved = [](double v, auto ctrl) {
+        union {
+            double d;
+            int i[2];
+        } u{v}, w;
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+            w.i[k] = __builtin_amdgcn_update_dpp(0, u.i[k], decltype(ctrl)::value, 0xF, 0xF, true);
+        return w.d;
+    };
+    x += moved(x, std::integral_constant<int, 0xB1>{});   // lanes 1 0 3 2 of each four
+    x += moved(x, std::integral_constant<int, 0x4E>{});   // lanes 2 3 0 1
+    x += moved(x, std::integral_constant<int, 0x141>{});  // the other four of each eight
+    x += moved(x, std::integral_constant<int, 0x140>{});  // the other eight
+    return x;
 }
 
-// q = K p over rows i = group, group + groups, ...; part[blockIdx.x] = this workgroup's
-// share of p.q. The columns are gathered from pm = P p (fixed dofs already zero), so a
-// block costs its own loads and one gather of pm; a fixed row takes p's own value. Every
-// lane of a row group runs the same trip count, so the butterfly always has its 16 lanes.
-template <bool ELA, int G>
-__global__ void __launch_bounds__(kBT)
-    k_spmv(const int *__restrict__ row, const int *__restrict__ col,
-           const double *__restrict__ values, const uint8_t *__restrict__ mask, int N,
-           const double *__restrict__ pm, const double *__restrict__ p, double *__restrict__ q,
-           double *__restrict__ part, const CgState *__restrict__ cs)
+// Fixed-order sums of NV values over a workgroup's kBT threads, on every thread; s: 4 NV
+// words of LDS.
+template <int NV>
+__device__ __forceinline__ void block_sums(double *s, double (&v)[NV])
 {
-    if (cs && cs->done) return;  // the whole grid returns: nothing waits on the butterfly
-    __shared__ double s[kBT];
-    constexpr int D = ELA ? 3 : 1;
-    const int l = threadIdx.x % G;
-    const int groups = gridDim.x * (kBT / G);
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        v[k] = row16_sum(v[k]);
+        v[k] += __shfl_xor(v[k], 16);
+        v[k] += __shfl_xor(v[k], 32);
+        if (lane == 0) s[4 * k + w] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = (s[4 * k] + s[4 * k + 1]) + (s[4 * k + 2] + s[4 * k + 3]);
+    __syncthreads();
+}
+
+// The sums of NV arrays of n partials (part, part + kMaxGrid, ...), on every thread.
+template <int NV>
+__device__ __forceinline__ void part_sums(double *s, const double *__restrict__ part, int n,
+                                          double (&v)[NV])
+{
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = 0.0;
+    for (int i = threadIdx.x; i < n; i += kBT)
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] += part[k * kMaxGrid + i];
+    block_sums<NV>(s, v);
+}
+
+// The lap product: q = K p over rows i = group, group + groups, ...; part[blockIdx.x] = this
+// workgroup's share of p.q. The columns are gathered from pm = P p (fixed dofs already zero),
+// so an entry costs its own load and one gather; a fixed row takes p's own value.
+__global__ void __launch_bounds__(kBT)
+    k_spmv_lap(const int *__restrict__ row, const int *__restrict__ col,
+               const double *__restrict__ values, const uint8_t *__restrict__ mask, int N,
+               const double *__restrict__ pm, const double *__restrict__ p, double *__restrict__ q,
+               double *__restrict__ part, const CgState *__restrict__ cs)
+{
+    if (cs && cs->done) return;
+    __shared__ double s[4];
+    const int l = threadIdx.x % kGroup;
+    const int groups = gridDim.x * (kBT / kGroup);
     double pq = 0.0;
-    for (int i = blockIdx.x * (kBT / G) + threadIdx.x / G; i < N; i += groups) {
+    for (int i = blockIdx.x * (kBT / kGroup) + threadIdx.x / kGroup; i < N; i += groups) {
         const int q0 = row[i], q1 = row[i + 1];
         const unsigned mi = mask[i];
-        double pi[D], acc[D];
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-            pi[d] = p[(int64_t)i * D + d];
-            acc[d] = 0.0;
-        }
-        for (int k = q0 + l; k < q1; k += G) {
-            const int j = col[k] - 1;
-            const double *b = values + (int64_t)k * D * D;
-            if constexpr (ELA) {
-                double v[9];
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const double2 w = *reinterpret_cast<const double2 *>(b + 2 * c);
-                    v[2 * c] = w.x;
-                    v[2 * c + 1] = w.y;
-                }
-                v[8] = b[8];
-                const double x0 = pm[(int64_t)j * 3], x1 = pm[(int64_t)j * 3 + 1],
-                             x2 = pm[(int64_t)j * 3 + 2];
-#pragma unroll
-                for (int d = 0; d < 3; d++) acc[d] += v[3 * d] * x0 + v[3 * d + 1] * x1 + v[3 * d + 2] * x2;
-            } else {
-                acc[0] += b[0] * pm[j];
-            }
-        }
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int d = 0; d < D; d++) acc[d] += __shfl_xor(acc[d], o, G);
+        const double pi = p[i];
+        double acc = 0.0;
+        for (int k = q0 + l; k < q1; k += kGroup) acc += values[k] * pm[col[k] - 1];
+        acc = row16_sum(acc);
         if (l == 0) {
-#pragma unroll
-            for (int d = 0; d < D; d++) {
-                const double qi = (mi >> d) & 1u ? pi[d] : acc[d];
-                q[(int64_t)i * D + d] = qi;
-                pq += pi[d] * qi;
-            }
+            const double qi = mi & 1u ? pi : acc;
+            q[i] = qi;
+            pq += pi * qi;
         }
     }
-    const double t = block_sum(s, pq);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+    double t[1] = {pq};
+    block_sums<1>(s, t);
+    if (threadIdx.x == 0) part[blockIdx.x] = t[0];
 }
 
 // The ela product with the value stream staged through LDS: a wave's four row groups own
@@ -161,7 +174,7 @@ __global__ void __launch_bounds__(kBT)
                       double *__restrict__ q, double *__restrict__ part, const CgState *__restrict__ cs)
 {
     if (cs && cs->done) return;
-    __shared__ double s[kBT];
+    __shared__ double s[4];
     __shared__ __align__(16) double stage[kBT / 64][kChunk * 9];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int l = lane & (kGroup - 1), g = lane / kGroup;
@@ -207,9 +220,7 @@ __global__ void __launch_bounds__(kBT)
             __builtin_amdgcn_wave_barrier();
         }
 #pragma unroll
-        for (int o = kGroup / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int d = 0; d < 3; d++) acc[d] += __shfl_xor(acc[d], o, kGroup);
+        for (int d = 0; d < 3; d++) acc[d] = row16_sum(acc[d]);
         if (l == 0 && on) {
 #pragma unroll
             for (int d = 0; d < 3; d++) {
@@ -219,248 +230,244 @@ __global__ void __launch_bounds__(kBT)
             }
         }
     }
-    const double t = block_sum(s, pq);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+    double t[1] = {pq};
+    block_sums<1>(s, t);
+    if (threadIdx.x == 0) part[blockIdx.x] = t[0];
 }
 
-// z = M r per node block; partA/partB[blockIdx.x] = this workgroup's share of r.z, r.r
+// z = M r of node i, from its residual; adds r.z and r.r to v[0] and v[1]
+template <bool ELA>
+__device__ __forceinline__ void prec_node(const double *__restrict__ prec, const uint8_t *__restrict__ mask,
+                                          int i, const double (&r)[ELA ? 3 : 1], double *__restrict__ z,
+                                          double &rz, double &rr)
+{
+    if constexpr (ELA) {
+        const double *m = prec + (int64_t)i * 9;
+        const double z0 = m[0] * r[0] + m[1] * r[1] + m[2] * r[2];
+        const double z1 = m[3] * r[0] + m[4] * r[1] + m[5] * r[2];
+        const double z2 = m[6] * r[0] + m[7] * r[1] + m[8] * r[2];
+        z[(int64_t)i * 3] = z0;
+        z[(int64_t)i * 3 + 1] = z1;
+        z[(int64_t)i * 3 + 2] = z2;
+        rz += r[0] * z0 + r[1] * z1 + r[2] * z2;
+        rr += r[0] * r[0] + r[1] * r[1] + r[2] * r[2];
+    } else {
+        // a masked lap node's row of K is the identity, so its prec is 1
+        const double zi = mask[i] ? r[0] : prec[i] * r[0];
+        z[i] = zi;
+        rz += r[0] * zi;
+        rr += r[0] * r[0];
+    }
+}
+
+// r = P b - q, z = M r; part: shares of r.z, r.r and (P b).(P b)
 template <bool ELA>
 __global__ void __launch_bounds__(kBT)
-    k_prec_dot(const double *__restrict__ prec, const uint8_t *__restrict__ mask, int N,
-               const double *__restrict__ r, double *__restrict__ z, double *__restrict__ partA,
-               double *__restrict__ partB)
+    k_start(const double *__restrict__ b, const double *__restrict__ q,
+            const double *__restrict__ prec, const uint8_t *__restrict__ mask, int N,
+            double *__restrict__ r, double *__restrict__ z, double *__restrict__ part)
 {
-    __shared__ double s[kBT];
-    double rz = 0.0, rr = 0.0;
+    constexpr int D = ELA ? 3 : 1;
+    __shared__ double s[12];
+    double v[3] = {0.0, 0.0, 0.0};
     for (int i = blockIdx.x * kBT + threadIdx.x; i < N; i += gridDim.x * kBT) {
-        if constexpr (ELA) {
-            const double *m = prec + (int64_t)i * 9;
-            const double r0 = r[(int64_t)i * 3], r1 = r[(int64_t)i * 3 + 1], r2 = r[(int64_t)i * 3 + 2];
-            const double z0 = m[0] * r0 + m[1] * r1 + m[2] * r2;
-            const double z1 = m[3] * r0 + m[4] * r1 + m[5] * r2;
-            const double z2 = m[6] * r0 + m[7] * r1 + m[8] * r2;
-            z[(int64_t)i * 3] = z0;
-            z[(int64_t)i * 3 + 1] = z1;
-            z[(int64_t)i * 3 + 2] = z2;
-            rz += r0 * z0 + r1 * z1 + r2 * z2;
-            rr += r0 * r0 + r1 * r1 + r2 * r2;
-        } else {
-            // a masked lap node's row of K is the identity, so its prec is 1
-            const double ri = r[i], zi = mask[i] ? ri : prec[i] * ri;
-            z[i] = zi;
-            rz += ri * zi;
-            rr += ri * ri;
-        }
-    }
-    const double a = block_sum(s, rz);
-    const double b = block_sum(s, rr);
-    if (threadIdx.x == 0) {
-        partA[blockIdx.x] = a;
-        partB[blockIdx.x] = b;
-    }
-}
-
-// out[k] = the fixed-order sum of part_k[0..n) (k < npart), one workgroup
-__global__ void __launch_bounds__(kBT)
-    k_sum_parts(const double *__restrict__ partA, const double *__restrict__ partB, int n,
-                double *__restrict__ out)
-{
-    __shared__ double s[kBT];
-    double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < n; i += kBT) {
-        a += partA[i];
-        if (partB) b += partB[i];
-    }
-    const double ta = block_sum(s, a);
-    const double tb = partB ? block_sum(s, b) : 0.0;
-    if (threadIdx.x == 0) {
-        out[0] = ta;
-        out[1] = tb;
-    }
-}
-
-// x += alpha p, r -= alpha q (alpha = r.z / p.q), then z = M r with the partial sums of
-// r.z and r.r: k_prec_dot on the updated residual, in the same grid and order
-template <bool ELA>
-__global__ void __launch_bounds__(kBT)
-    k_update_prec_dot(const CgState *__restrict__ cs, const double *__restrict__ p,
-                      const double *__restrict__ q, double *__restrict__ x, double *__restrict__ r,
-                      const double *__restrict__ prec, const uint8_t *__restrict__ mask, int N,
-                      double *__restrict__ z, double *__restrict__ partA, double *__restrict__ partB)
-{
-    if (cs->done) return;
-    __shared__ double s[kBT];
-    const double alpha = cs->rz / cs->pq;
-    double rz = 0.0, rr = 0.0;
-    for (int i = blockIdx.x * kBT + threadIdx.x; i < N; i += gridDim.x * kBT) {
-        if constexpr (ELA) {
-            double rv[3];
+        const unsigned mi = mask[i];
+        double rv[D];
 #pragma unroll
-            for (int d = 0; d < 3; d++) {
-                const int64_t k = (int64_t)i * 3 + d;
-                x[k] += alpha * p[k];
-                rv[d] = r[k] - alpha * q[k];
-                r[k] = rv[d];
-            }
-            const double *m = prec + (int64_t)i * 9;
-            const double z0 = m[0] * rv[0] + m[1] * rv[1] + m[2] * rv[2];
-            const double z1 = m[3] * rv[0] + m[4] * rv[1] + m[5] * rv[2];
-            const double z2 = m[6] * rv[0] + m[7] * rv[1] + m[8] * rv[2];
-            z[(int64_t)i * 3] = z0;
-            z[(int64_t)i * 3 + 1] = z1;
-            z[(int64_t)i * 3 + 2] = z2;
-            rz += rv[0] * z0 + rv[1] * z1 + rv[2] * z2;
-            rr += rv[0] * rv[0] + rv[1] * rv[1] + rv[2] * rv[2];
-        } else {
-            x[i] += alpha * p[i];
-            const double ri = r[i] - alpha * q[i];
-            r[i] = ri;
-            const double zi = mask[i] ? ri : prec[i] * ri;
-            z[i] = zi;
-            rz += ri * zi;
-            rr += ri * ri;
+        for (int d = 0; d < D; d++) {
+            const int64_t k = (int64_t)i * D + d;
+            const double bi = (mi >> d) & 1u ? 0.0 : b[k];
+            rv[d] = bi - q[k];
+            r[k] = rv[d];
+            v[2] += bi * bi;
         }
+        prec_node<ELA>(prec, mask, i, rv, z, v[0], v[1]);
     }
-    const double a = block_sum(s, rz);
-    const double b = block_sum(s, rr);
-    if (threadIdx.x == 0) {
-        partA[blockIdx.x] = a;
-        partB[blockIdx.x] = b;
-    }
+    block_sums<3>(s, v);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 3; k++) part[k * kMaxGrid + blockIdx.x] = v[k];
 }
 
-// the iteration's p.q from the spmv partials; p.q <= 0 stops the iteration before x moves
-__global__ void __launch_bounds__(kBT) k_sum_pq(const double *__restrict__ part, int n, CgState *cs)
-{
-    if (cs->done) return;
-    __shared__ double s[kBT];
-    double a = 0.0;
-    for (int i = threadIdx.x; i < n; i += kBT) a += part[i];
-    const double t = block_sum(s, a);
-    if (threadIdx.x == 0) {
-        cs->pq = t;
-        if (!(t > 0.0)) cs->done = 2;  // K is not positive definite on p (or p = 0)
-    }
-}
-
-// r.z and r.r of the updated residual from the partials, and the end of the iteration:
-// beta = r.z (new) / r.z (old) for the direction update, the new r.z becomes the old one,
-// and the solve stops at max_it or convergence (the direction update is then not needed)
+// x += alpha p, r -= alpha q (alpha = r.z / p.q, from the product's partials), then z = M r;
+// part: shares of r.z and r.r. p.q <= 0 stops the iteration before x moves.
+template <bool ELA>
 __global__ void __launch_bounds__(kBT)
-    k_sum_rz(const double *__restrict__ partA, const double *__restrict__ partB, int n, CgState *cs)
+    k_update_prec_dot(const CgState *__restrict__ cs, const double *__restrict__ pqPart, int nPart,
+                      const double *__restrict__ p, const double *__restrict__ q,
+                      double *__restrict__ x, double *__restrict__ r,
+                      const double *__restrict__ prec, const uint8_t *__restrict__ mask, int N,
+                      double *__restrict__ z, double *__restrict__ part, int *__restrict__ broken)
 {
+    constexpr int D = ELA ? 3 : 1;
     if (cs->done) return;
-    __shared__ double s[kBT];
-    double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < n; i += kBT) {
-        a += partA[i];
-        b += partB[i];
+    __shared__ double s[8];
+    double pq[1];
+    part_sums<1>(s, pqPart, nPart, pq);
+    if (!(pq[0] > 0.0)) {  // K is not positive definite on p (or p = 0)
+        if (blockIdx.x == 0 && threadIdx.x == 0) *broken = 1;
+        return;
     }
-    const double ta = block_sum(s, a);
-    const double tb = block_sum(s, b);
-    if (threadIdx.x == 0) {
-        cs->rz1 = ta;
-        cs->rr = tb;
-        cs->beta = ta / cs->rz;
-        cs->rz = ta;
-        cs->it += 1;
-        if (cs->it >= cs->max_it || !(sqrt(tb) > cs->tol)) cs->done = 1;
+    const double alpha = cs->rz / pq[0];
+    double v[2] = {0.0, 0.0};
+    for (int i = blockIdx.x * kBT + threadIdx.x; i < N; i += gridDim.x * kBT) {
+        double rv[D];
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            const int64_t k = (int64_t)i * D + d;
+            x[k] += alpha * p[k];
+            rv[d] = r[k] - alpha * q[k];
+            r[k] = rv[d];
+        }
+        prec_node<ELA>(prec, mask, i, rv, z, v[0], v[1]);
     }
+    block_sums<2>(s, v);
+    if (threadIdx.x == 0)
+        for (int k = 0; k < 2; k++) part[k * kMaxGrid + blockIdx.x] = v[k];
 }
 
-// p = z + beta p and pm = P p; without a state: p = z, whatever p held before
-__global__ void k_xpby(const double *__restrict__ z, const CgState *__restrict__ cs,
-                       const uint8_t *__restrict__ mask, int D, double *__restrict__ p,
-                       double *__restrict__ pm, int64_t n)
-{
-    if (cs && cs->done) return;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double v = cs ? z[i] + cs->beta * p[i] : z[i];
-    p[i] = v;
-    pm[i] = (mask[i / D] >> (i % D)) & 1u ? 0.0 : v;
-}
-
-// rhs = P b (fixed dofs set to 0); r = rhs - q; partA/partB: shares of rhs.rhs
+// The end of an iteration: r.z and r.r of the updated residual from the partials, beta = r.z
+// (new) / r.z (old), the next state (the solve stops at max_it or convergence), and, when it
+// goes on, p = z + beta p and pm = P p (pm may be null). Without a state cs (the start): p = z
+// and the first state, from k_start's partials, h its constants.
 __global__ void __launch_bounds__(kBT)
-    k_residual0(const double *__restrict__ b, const uint8_t *__restrict__ mask, int D,
-                const double *__restrict__ q, double *__restrict__ rhs, double *__restrict__ r,
-                int64_t n, double *__restrict__ part)
+    k_direction(const CgState *__restrict__ cs, CgState h, CgState *__restrict__ next, double rtol,
+                const double *__restrict__ part, int nPart, const int *__restrict__ broken,
+                const double *__restrict__ z, const uint8_t *__restrict__ mask, int D,
+                double *__restrict__ p, double *__restrict__ pm, int64_t n)
 {
-    __shared__ double s[kBT];
-    double bb = 0.0;
+    __shared__ double s[12];
+    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+    double beta = 0.0;
+    if (cs) {
+        h = *cs;
+        if (h.done || *broken) {
+            if (first) {
+                if (!h.done) h.done = 2;
+                *next = h;
+            }
+            return;
+        }
+        double v[2];
+        part_sums<2>(s, part, nPart, v);
+        beta = v[0] / h.rz;
+        h.rz = v[0];
+        h.rr = v[1];
+        h.it += 1;
+        h.done = h.it >= h.max_it || !(sqrt(h.rr) > h.tol) ? 1 : 0;
+    } else {
+        double v[3];
+        part_sums<3>(s, part, nPart, v);
+        h.rz = v[0];
+        h.rr = v[1];
+        h.bnorm = sqrt(v[2]) > 0.0 ? sqrt(v[2]) : 1.0;
+        h.tol = rtol * h.bnorm;
+        h.it = 0;
+        h.done = h.max_it > 0 && sqrt(h.rr) > h.tol ? 0 : 1;
+    }
+    if (first) *next = h;
+    if (h.done) return;
     for (int64_t i = (int64_t)blockIdx.x * kBT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBT) {
-        const int node = (int)(i / D), d = (int)(i % D);
-        const double v = (mask[node] >> d) & 1u ? 0.0 : b[i];
-        rhs[i] = v;
-        r[i] = v - q[i];
-        bb += v * v;
+        const double v = cs ? z[i] + beta * p[i] : z[i];
+        p[i] = v;
+        if (pm) pm[i] = (mask[i / D] >> (i % D)) & 1u ? 0.0 : v;
     }
-    const double t = block_sum(s, bb);
-    if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+// pm = P x
+__global__ void __launch_bounds__(kBT)
+    k_masked(const double *__restrict__ x, const uint8_t *__restrict__ mask, int D,
+             double *__restrict__ pm, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * kBT + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBT)
+        pm[i] = (mask[i / D] >> (i % D)) & 1u ? 0.0 : x[i];
 }
 
 // ---- the system in another node order (mf_pcg_ordered)
 
-// flag = 1 when some order[t] lies outside [0, N)
-__global__ void k_order_range(const int *__restrict__ order, int N, int *flag)
+// inv[order[t]] = t; flag = 1 when some order[t] lies outside [0, N)
+__global__ void k_order_invert(const int *__restrict__ order, int N, int *__restrict__ inv, int *flag)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < N && (order[t] < 0 || order[t] >= N)) atomicOr(flag, 1);
+    if (t >= N) return;
+    const int i = order[t];
+    if (i < 0 || i >= N) *flag = 1;
+    else inv[i] = t;
 }
 
-__global__ void k_order_invert(const int *__restrict__ order, int N, int *__restrict__ inv)
+// len[t] = length of row order[t]; len[N] = 0 (the exclusive scan then ends in nnz); flag = 1
+// for a negative length and when order repeats a node (some inv[order[t]] then names another t)
+__global__ void k_order_rowlen(const int *__restrict__ order, const int *__restrict__ inv,
+                               const int *__restrict__ row, int N, int *__restrict__ len, int *flag)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < N) inv[order[t]] = t;
-}
-
-// flag = 1 when order repeats a node (then some inv[order[t]] names another t)
-__global__ void k_order_dups(const int *__restrict__ order, const int *__restrict__ inv, int N, int *flag)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < N && inv[order[t]] != t) atomicOr(flag, 1);
-}
-
-// len[t] = length of row order[t]; len[N] = 0 (the exclusive scan then ends in nnz);
-// flag = 1 for a negative length
-__global__ void k_order_rowlen(const int *__restrict__ order, const int *__restrict__ row, int N,
-                               int *__restrict__ len, int *flag)
-{
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t > N) return;
+    int l = 0;
     if (t < N) {
-        const int l = row[order[t] + 1] - row[order[t]];
-        len[t] = l;
-        if (l < 0) atomicOr(flag, 1);
-    } else if (t == N) {
-        len[t] = 0;
+        const int i = order[t];
+        if (i >= 0 && i < N) {
+            l = row[i + 1] - row[i];
+            if (l < 0 || inv[i] != t) *flag = 1;
+        }
     }
+    len[t] = l;
 }
 
 // flag = 1 for a column outside 1..N
 __global__ void k_check_cols(const int *__restrict__ col, int64_t nnz, int N, int *flag)
 {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nnz && (col[k] < 1 || col[k] > N)) atomicOr(flag, 1);
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < nnz; k += stride)
+        if (col[k] < 1 || col[k] > N) *flag = 1;
 }
 
-// new row t = old row order[t], its entries in their own order, columns renumbered
+// New row t = old row order[t], its entries in their own order, columns renumbered, the
+// columns of fixed dofs zero (m: the mask in the new order): the product then gathers the
+// direction itself, and needs no masked copy of it. A row's values are one contiguous run on
+// both sides, moved by its 16 lanes in 16-byte pieces, five of a lane in flight (333 us for
+// ela 80^3, a block per lane word by word 386: rows of 1 KB in random order); the few columns
+// of fixed dofs are zeroed after them, by the same wave.
 template <int DD>
 __global__ void __launch_bounds__(kBT)
     k_order_csr(const int *__restrict__ order, const int *__restrict__ inv,
                 const int *__restrict__ row, const int *__restrict__ col,
-                const double *__restrict__ values, const int *__restrict__ rowp, int N,
-                int *__restrict__ colp, double *__restrict__ valp)
+                const double *__restrict__ values, const int *__restrict__ rowp,
+                const uint8_t *__restrict__ m, int N, int *__restrict__ colp,
+                double *__restrict__ valp)
 {
+    constexpr int CP = 5;
     const int l = threadIdx.x % kGroup;
     const int groups = gridDim.x * (kBT / kGroup);
     for (int t = blockIdx.x * (kBT / kGroup) + threadIdx.x / kGroup; t < N; t += groups) {
-        const int i = order[t], src = row[i], len = row[i + 1] - src, dst = rowp[t];
-        for (int k = l; k < len; k += kGroup) {
-            colp[dst + k] = inv[col[src + k] - 1] + 1;
+        const int i = order[t], src = row[i], n = row[i + 1] - src, dst = rowp[t], nd = n * DD;
+        const double *from = values + (int64_t)src * DD;
+        double *to = valp + (int64_t)dst * DD;
+        for (int j0 = 2 * l; j0 < nd; j0 += 2 * kGroup * CP) {
+            double2 v[CP];
 #pragma unroll
-            for (int w = 0; w < DD; w++)
-                valp[(int64_t)(dst + k) * DD + w] = values[(int64_t)(src + k) * DD + w];
+            for (int k = 0; k < CP; k++) {
+                const int j = j0 + 2 * kGroup * k;
+                if (j + 1 < nd) v[k] = *reinterpret_cast<const double2 *>(from + j);
+                else if (j < nd) v[k].x = from[j];
+            }
+#pragma unroll
+            for (int k = 0; k < CP; k++) {
+                const int j = j0 + 2 * kGroup * k;
+                if (j + 1 < nd) *reinterpret_cast<double2 *>(to + j) = v[k];
+                else if (j < nd) to[j] = v[k].x;
+            }
+        }
+        for (int k = l; k < n; k += kGroup) {
+            const int j = inv[col[src + k] - 1];
+            colp[dst + k] = j + 1;
+            const unsigned mj = m[j];
+            if (!mj) continue;
+            double *o = to + (int64_t)k * DD;
+            if constexpr (DD == 9) {
+                for (int e = 0; e < 3; e++)
+                    if ((mj >> e) & 1u) o[e] = o[3 + e] = o[6 + e] = 0.0;
+            } else {
+                o[0] = 0.0;
+            }
         }
     }
 }
@@ -481,134 +488,76 @@ inline int grid_for(int64_t items) { return (int)std::max<int64_t>(1, std::min<i
 
 }  // namespace
 
-// The solve on one numbering of the nodes; order (may be NULL) maps it to checkBounds'
-// (entry t of every array is node order[t]).
-static int pcg_core(bool ela, int nbNodes, const int *row, const int *col, const double *values,
-             const double *prec, const int *checkBounds, const int *order, const double *b,
-             double *x, double rtol, int maxIter, int *iterations, double *relResidual,
-             hipStream_t s)
+// The solve on one numbering of the nodes. copied: the system is k_order_csr's copy, whose
+// columns of fixed dofs are zero, so the direction itself takes the place of its masked copy.
+static int pcg_core(bool ela, bool copied, int nbNodes, const int *row, const int *col,
+                    const double *values, const double *prec, const uint8_t *mask,
+                    const double *b, double *x, double rtol, int maxIter, int *iterations,
+                    double *relResidual, hipStream_t s)
 {
     const int D = ela ? 3 : 1;
     const int64_t n = (int64_t)nbNodes * D;
-    if (iterations) *iterations = 0;
-    if (relResidual) *relResidual = 0.0;
-    if (n == 0) return MF_OK;
-    // r, z, p, q, rhs, pm = P p; partials (2 x kMaxGrid); the two sums; the state; the
-    // mask bytes
-    const size_t vec = (size_t)n * sizeof(double);
-    const size_t bytes = 6 * vec + 2 * kMaxGrid * sizeof(double) + 2 * sizeof(double) +
-                         sizeof(CgState) + (size_t)nbNodes;
-    unsigned char *buf = nullptr;
-    if (hipMalloc(&buf, bytes) != hipSuccess) return MF_ERR_NOMEM;
-    double *r = reinterpret_cast<double *>(buf), *z = r + n, *p = z + n, *q = p + n, *rhs = q + n;
-    double *pm = rhs + n, *partA = pm + n, *partB = partA + kMaxGrid, *sums = partB + kMaxGrid;
-    CgState *cs = reinterpret_cast<CgState *>(sums + 2);
-    uint8_t *mask = reinterpret_cast<uint8_t *>(cs + 1);
+    // r, z, p, q, pm = P p (not for a copy); 1 + 3 arrays of kMaxGrid partials; two states;
+    // the breakdown flag
+    const size_t vec = mf::Workspace::padded((size_t)n * sizeof(double));
+    mf::Workspace ws((copied ? 4 : 5) * vec + mf::Workspace::padded(4 * kMaxGrid * sizeof(double)) +
+                         mf::Workspace::padded(2 * sizeof(CgState)) + mf::Workspace::padded(sizeof(int)), s);
+    if (!ws.ok()) return MF_ERR_NOMEM;
+    double *r = ws.cut<double>(n), *z = ws.cut<double>(n), *p = ws.cut<double>(n), *q = ws.cut<double>(n);
+    double *pm = copied ? nullptr : ws.cut<double>(n);
+    double *pqPart = ws.cut<double>(4 * kMaxGrid), *part = pqPart + kMaxGrid;
+    CgState *cs = ws.cut<CgState>(2);
+    int *broken = ws.cut<int>(1);
     const int gSpmv = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ((int64_t)nbNodes * kGroup + kBT - 1) / kBT));
-    const int gSpmvLap = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ((int64_t)nbNodes * kLapGroup + kBT - 1) / kBT));
     const int gNode = grid_for(nbNodes), gDof = grid_for(n);
-    int st = MF_OK;
-    auto launched = [&]() {
-        if (st == MF_OK && hipGetLastError() != hipSuccess) st = MF_ERR_HIP;
-        return st == MF_OK;
-    };
     // out = K in, from in and its masked copy in_m (state: skipped once the solve is done)
     auto spmv = [&](const double *in_m, const double *in, double *out, const CgState *c) {
-        if (ela)
-            hipLaunchKernelGGL(k_spmv_ela_staged, dim3(gSpmv), dim3(kBT), 0, s, row, col, values,
-                               mask, nbNodes, in_m, in, out, partA, c);
-        else
-            hipLaunchKernelGGL((k_spmv<false, kLapGroup>), dim3(gSpmvLap), dim3(kBT), 0, s, row, col,
-                               values, mask, nbNodes, in_m, in, out, partA, c);
+        auto kern = ela ? k_spmv_ela_staged : k_spmv_lap;
+        hipLaunchKernelGGL(kern, dim3(gSpmv), dim3(kBT), 0, s, row, col, values, mask, nbNodes,
+                           copied ? in : in_m, in, out, pqPart, c);
     };
-    // p = z (c NULL) or p = z + beta p, and pm = P p
-    auto xpby = [&](const CgState *c) {
-        hipLaunchKernelGGL(k_xpby, g1(n), dim3(kBT), 0, s, z, c, mask, D, p, pm, n);
-    };
-    auto prec_dot = [&]() {
-        if (ela)
-            hipLaunchKernelGGL(k_prec_dot<true>, dim3(gNode), dim3(kBT), 0, s, prec, mask, nbNodes, r,
-                               z, partA, partB);
-        else
-            hipLaunchKernelGGL(k_prec_dot<false>, dim3(gNode), dim3(kBT), 0, s, prec, mask, nbNodes,
-                               r, z, partA, partB);
-    };
-    // the two sums of the partials of a grid of g workgroups, on the host
-    double h2[2] = {0.0, 0.0};
-    auto sums_of = [&](int g, bool two) {
-        hipLaunchKernelGGL(k_sum_parts, dim3(1), dim3(kBT), 0, s, partA, two ? partB : nullptr, g,
-                           sums);
-        if (!launched()) return false;
-        if (hipMemcpyAsync(h2, sums, sizeof(h2), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            st = MF_ERR_HIP;
-        return st == MF_OK;
-    };
-
-    // rhs = P b; r = rhs - K x; z = M r; p = z
-    hipLaunchKernelGGL(k_mask_bits, g1(nbNodes), dim3(kBT), 0, s, checkBounds, nbNodes, ela, order,
-                       mask);
-    launched();
-    double bnorm2 = 0.0, rz = 0.0, rr = 0.0;
-    if (st == MF_OK) {
-        // p = x, pm = P x: scratch for q = K x
-        hipLaunchKernelGGL(k_xpby, g1(n), dim3(kBT), 0, s, x, nullptr, mask, D, p, pm, n);
-        spmv(pm, p, q, nullptr);  // its p.q partials are not used
-        hipLaunchKernelGGL(k_residual0, dim3(gDof), dim3(kBT), 0, s, b, mask, D, q, rhs, r, n,
-                           partA);
-        if (launched() && sums_of(gDof, false)) bnorm2 = h2[0];
-    }
-    if (st == MF_OK) {
-        prec_dot();
-        if (launched() && sums_of(gNode, true)) {
-            rz = h2[0];
-            rr = h2[1];
-        }
-    }
-    if (st == MF_OK) {
-        xpby(nullptr);  // p = z
-        launched();
-    }
-    const double bnorm = std::sqrt(bnorm2) > 0.0 ? std::sqrt(bnorm2) : 1.0;
-    // the iterations, enqueued kBatch at a time; k_sum_rz counts each one and decides, as
-    // the loop condition would, whether another one runs
     CgState h{};
-    h.rz = rz;
-    h.rz1 = rz;
-    h.rr = rr;
-    h.tol = rtol * bnorm;
-    h.it = 0;
     h.max_it = maxIter;
-    h.done = maxIter > 0 && std::sqrt(rr) > h.tol ? 0 : 1;
-    if (st == MF_OK && (hipMemcpyAsync(cs, &h, sizeof(h), hipMemcpyHostToDevice, s) != hipSuccess ||
-                        hipStreamSynchronize(s) != hipSuccess))
-        st = MF_ERR_HIP;
-    while (st == MF_OK && !h.done) {
-        for (int k = 0; k < kBatch; k++) {
-            spmv(pm, p, q, cs);
-            hipLaunchKernelGGL(k_sum_pq, dim3(1), dim3(kBT), 0, s, partA, ela ? gSpmv : gSpmvLap, cs);
+    auto direction = [&](const CgState *c, CgState *next) {
+        hipLaunchKernelGGL(k_direction, dim3(gDof), dim3(kBT), 0, s, c, h, next, rtol, part, gNode,
+                           broken, z, mask, D, p, pm, n);
+    };
+    // r = P b - K x; z = M r; p = z
+    const int zero = 0;
+    if (hipMemcpyAsync(broken, &zero, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess) return MF_ERR_HIP;
+    if (!copied) hipLaunchKernelGGL(k_masked, dim3(gDof), dim3(kBT), 0, s, x, mask, D, pm, n);
+    spmv(pm, x, q, nullptr);  // its p.q partials are not used
+    if (ela)
+        hipLaunchKernelGGL(k_start<true>, dim3(gNode), dim3(kBT), 0, s, b, q, prec, mask, nbNodes, r, z, part);
+    else
+        hipLaunchKernelGGL(k_start<false>, dim3(gNode), dim3(kBT), 0, s, b, q, prec, mask, nbNodes, r, z, part);
+    direction(nullptr, cs);
+    // the iterations, enqueued kBatch at a time; k_direction counts each one and decides, as
+    // the loop condition would, whether another one runs
+    int done = 0, sent = 0;
+    do {
+        for (int k = 0; k < kBatch && sent < maxIter; k++, sent++) {
+            const CgState *c = cs + (sent & 1);
+            spmv(pm, p, q, c);
             if (ela)
-                hipLaunchKernelGGL(k_update_prec_dot<true>, dim3(gNode), dim3(kBT), 0, s, cs, p, q,
-                                   x, r, prec, mask, nbNodes, z, partA, partB);
+                hipLaunchKernelGGL(k_update_prec_dot<true>, dim3(gNode), dim3(kBT), 0, s, c, pqPart,
+                                   gSpmv, p, q, x, r, prec, mask, nbNodes, z, part, broken);
             else
-                hipLaunchKernelGGL(k_update_prec_dot<false>, dim3(gNode), dim3(kBT), 0, s, cs, p, q,
-                                   x, r, prec, mask, nbNodes, z, partA, partB);
-            hipLaunchKernelGGL(k_sum_rz, dim3(1), dim3(kBT), 0, s, partA, partB, gNode, cs);
-            xpby(cs);
+                hipLaunchKernelGGL(k_update_prec_dot<false>, dim3(gNode), dim3(kBT), 0, s, c, pqPart,
+                                   gSpmv, p, q, x, r, prec, mask, nbNodes, z, part, broken);
+            direction(c, cs + ((sent + 1) & 1));
         }
-        if (!launched()) break;
-        if (hipMemcpyAsync(&h, cs, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess)
-            st = MF_ERR_HIP;
-    }
-    const int it = h.it;
-    rr = h.rr;
-    if (st == MF_OK && hipStreamSynchronize(s) != hipSuccess) st = MF_ERR_HIP;
-    if (iterations) *iterations = it;
-    if (relResidual) *relResidual = std::sqrt(rr) / bnorm;
-    (void)hipStreamSynchronize(s);  // nothing in flight reads buf when it is freed
-    (void)hipFree(buf);
-    return st;
+        if (hipGetLastError() != hipSuccess ||
+            hipMemcpyAsync(&h, cs + (sent & 1), sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            return MF_ERR_HIP;
+        }
+        done = h.done;
+    } while (!done);
+    if (iterations) *iterations = h.it;
+    if (relResidual) *relResidual = std::sqrt(h.rr) / h.bnorm;
+    return MF_OK;
 }
 
 extern "C" int mf_pcg(int operatorID, int nbNodes, const int *row, const int *col,
@@ -620,8 +569,17 @@ extern "C" int mf_pcg(int operatorID, int nbNodes, const int *row, const int *co
     if ((operatorID != MF_OP_LAP && !ela) || nbNodes < 0 || !row || !values || !prec || !b || !x ||
         maxIter < 0 || !(rtol > 0.0))
         return MF_ERR_ARG;
-    return pcg_core(ela, nbNodes, row, col, values, prec, checkBounds, nullptr, b, x, rtol, maxIter,
-                    iterations, relResidual, reinterpret_cast<hipStream_t>(stream));
+    if (iterations) *iterations = 0;
+    if (relResidual) *relResidual = 0.0;
+    if (nbNodes == 0) return MF_OK;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    mf::Workspace ws(mf::Workspace::padded((size_t)nbNodes), s);
+    if (!ws.ok()) return MF_ERR_NOMEM;
+    uint8_t *mask = ws.cut<uint8_t>(nbNodes);
+    hipLaunchKernelGGL(k_mask_bits, g1(nbNodes), dim3(kBT), 0, s, checkBounds, nbNodes, ela,
+                       (const int *)nullptr, mask);
+    return pcg_core(ela, false, nbNodes, row, col, values, prec, mask, b, x, rtol, maxIter, iterations,
+                    relResidual, s);
 }
 
 extern "C" int mf_pcg_ordered(int operatorID, int nbNodes, const int *row, const int *col,
@@ -649,86 +607,55 @@ extern "C" int mf_pcg_ordered(int operatorID, int nbNodes, const int *row, const
     if (hipcub::DeviceScan::ExclusiveSum(nullptr, scan_bytes, (const int *)nullptr, (int *)nullptr,
                                          N + 1, s) != hipSuccess)
         return MF_ERR_HIP;
-    // flag, inv[N], len[N+1], rowp[N+1], colp[nnz], valp[nnz DD], precp[N DD], bp, xp[N D],
-    // the scan's scratch; each piece 256-byte aligned
-    auto al = [](size_t v) { return (v + 255) / 256 * 256; };
-    const size_t o_inv = 256, o_len = o_inv + al(4 * (size_t)N), o_rowp = o_len + al(4 * ((size_t)N + 1)),
-                 o_col = o_rowp + al(4 * ((size_t)N + 1)), o_val = o_col + al(4 * (size_t)nnz),
-                 o_prec = o_val + al(8 * (size_t)nnz * DD), o_b = o_prec + al(8 * (size_t)N * DD),
-                 o_x = o_b + al(8 * (size_t)N * D), o_scan = o_x + al(8 * (size_t)N * D),
-                 bytes = o_scan + al(scan_bytes);
-    unsigned char *buf = nullptr;
-    if (hipMalloc(&buf, bytes) != hipSuccess) return MF_ERR_NOMEM;
-    int *flag = reinterpret_cast<int *>(buf), *inv = reinterpret_cast<int *>(buf + o_inv),
-        *len = reinterpret_cast<int *>(buf + o_len), *rowp = reinterpret_cast<int *>(buf + o_rowp),
-        *colp = reinterpret_cast<int *>(buf + o_col);
-    double *valp = reinterpret_cast<double *>(buf + o_val), *precp = reinterpret_cast<double *>(buf + o_prec),
-           *bp = reinterpret_cast<double *>(buf + o_b), *xp = reinterpret_cast<double *>(buf + o_x);
-    int st = MF_OK;
-    auto launched = [&]() {
-        if (st == MF_OK && hipGetLastError() != hipSuccess) st = MF_ERR_HIP;
-        return st == MF_OK;
-    };
+    const auto pad = [](size_t v) { return mf::Workspace::padded(v); };
+    mf::Workspace ws(256 + pad(4 * (size_t)N) + 2 * pad(4 * ((size_t)N + 1)) + pad(4 * (size_t)nnz) +
+                         pad(8 * (size_t)nnz * DD) + pad(8 * (size_t)N * DD) +
+                         2 * pad(8 * (size_t)N * D) + pad((size_t)N) + pad(scan_bytes + 1), s);
+    if (!ws.ok()) return MF_ERR_NOMEM;
+    int *flag = ws.cut<int>(1), *inv = ws.cut<int>(N), *len = ws.cut<int>((size_t)N + 1),
+        *rowp = ws.cut<int>((size_t)N + 1), *colp = ws.cut<int>(nnz);
+    double *valp = ws.cut<double>((size_t)nnz * DD), *precp = ws.cut<double>((size_t)N * DD),
+           *bp = ws.cut<double>((size_t)N * D), *xp = ws.cut<double>((size_t)N * D);
+    uint8_t *mask = ws.cut<uint8_t>(N);
+    void *scan = ws.cut<unsigned char>(scan_bytes + 1);
     // the copies below write where row and order say: order must be a permutation of
-    // 0..N-1 (every index in range first, then no repeats), every row length >= 0 (with
-    // row[0] = 0 and row[N] = nnz, each new row then lies inside 0..nnz) and every column
-    // in 1..N
-    auto flag_set = [&]() {
-        int h = 0;
-        if (hipMemcpyAsync(&h, flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess) {
-            st = MF_ERR_HIP;
-            return true;
-        }
-        return h != 0;
-    };
-    const int zero = 0;
-    if (hipMemcpyAsync(flag, &zero, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess)
-        st = MF_ERR_HIP;
-    if (st == MF_OK) {
-        hipLaunchKernelGGL(k_order_range, g1(N), dim3(kBT), 0, s, order, N, flag);
-        if (launched() && flag_set() && st == MF_OK) st = MF_ERR_ARG;
-    }
-    if (st == MF_OK) {
-        hipLaunchKernelGGL(k_order_invert, g1(N), dim3(kBT), 0, s, order, N, inv);
-        hipLaunchKernelGGL(k_order_dups, g1(N), dim3(kBT), 0, s, order, inv, N, flag);
-        if (launched() && flag_set() && st == MF_OK) st = MF_ERR_ARG;
-    }
-    if (st == MF_OK) {
-        hipLaunchKernelGGL(k_order_rowlen, g1((int64_t)N + 1), dim3(kBT), 0, s, order, row, N, len,
-                           flag);
-        if (nnz > 0)
-            hipLaunchKernelGGL(k_check_cols, g1(nnz), dim3(kBT), 0, s, col, (int64_t)nnz, N, flag);
-        if (launched() && flag_set() && st == MF_OK) st = MF_ERR_ARG;
-    }
-    if (st == MF_OK && hipcub::DeviceScan::ExclusiveSum(buf + o_scan, scan_bytes, len, rowp, N + 1,
-                                                        s) != hipSuccess)
-        st = MF_ERR_HIP;
-    if (st == MF_OK) {
-        const int g = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ((int64_t)N * kGroup + kBT - 1) / kBT));
-        if (ela)
-            hipLaunchKernelGGL(k_order_csr<9>, dim3(g), dim3(kBT), 0, s, order, inv, row, col, values,
-                               rowp, N, colp, valp);
-        else
-            hipLaunchKernelGGL(k_order_csr<1>, dim3(g), dim3(kBT), 0, s, order, inv, row, col, values,
-                               rowp, N, colp, valp);
-        hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * DD), dim3(kBT), 0, s, order, (int64_t)N * DD,
-                           DD, true, prec, precp);
-        hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * D), dim3(kBT), 0, s, order, (int64_t)N * D, D,
-                           true, b, bp);
-        hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * D), dim3(kBT), 0, s, order, (int64_t)N * D, D,
-                           true, x, xp);
-        launched();
-    }
+    // 0..N-1 (every index in range, no repeats), every row length >= 0 (with row[0] = 0 and
+    // row[N] = nnz, each new row then lies inside 0..nnz) and every column in 1..N
+    int bad = 0;
+    if (hipMemcpyAsync(flag, &bad, sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess) return MF_ERR_HIP;
+    hipLaunchKernelGGL(k_order_invert, g1(N), dim3(kBT), 0, s, order, N, inv, flag);
+    hipLaunchKernelGGL(k_order_rowlen, g1((int64_t)N + 1), dim3(kBT), 0, s, order, inv, row, N, len, flag);
+    if (nnz > 0)
+        hipLaunchKernelGGL(k_check_cols, dim3(grid_for(nnz)), dim3(kBT), 0, s, col, (int64_t)nnz, N, flag);
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return MF_ERR_HIP;
+    if (bad) return MF_ERR_ARG;
+    if (hipcub::DeviceScan::ExclusiveSum(scan, scan_bytes, len, rowp, N + 1, s) != hipSuccess)
+        return MF_ERR_HIP;
+    hipLaunchKernelGGL(k_mask_bits, g1(N), dim3(kBT), 0, s, checkBounds, N, ela, order, mask);
+    const int g = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxGrid, ((int64_t)N * kGroup + kBT - 1) / kBT));
+    if (ela)
+        hipLaunchKernelGGL(k_order_csr<9>, dim3(g), dim3(kBT), 0, s, order, inv, row, col, values,
+                           rowp, mask, N, colp, valp);
+    else
+        hipLaunchKernelGGL(k_order_csr<1>, dim3(g), dim3(kBT), 0, s, order, inv, row, col, values,
+                           rowp, mask, N, colp, valp);
+    hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * DD), dim3(kBT), 0, s, order, (int64_t)N * DD, DD,
+                       true, prec, precp);
+    hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * D), dim3(kBT), 0, s, order, (int64_t)N * D, D,
+                       true, b, bp);
+    hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * D), dim3(kBT), 0, s, order, (int64_t)N * D, D,
+                       true, x, xp);
+    int st = hipGetLastError() == hipSuccess ? MF_OK : MF_ERR_HIP;
     if (st == MF_OK)
-        st = pcg_core(ela, N, rowp, colp, valp, precp, checkBounds, order, bp, xp, rtol, maxIter,
-                      iterations, relResidual, s);
+        st = pcg_core(ela, true, N, rowp, colp, valp, precp, mask, bp, xp, rtol, maxIter, iterations,
+                      relResidual, s);
     if (st == MF_OK) {
         hipLaunchKernelGGL(k_order_rows, g1((int64_t)N * D), dim3(kBT), 0, s, order, (int64_t)N * D, D,
                            false, xp, x);
-        if (launched() && hipStreamSynchronize(s) != hipSuccess) st = MF_ERR_HIP;
+        if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) st = MF_ERR_HIP;
     }
-    (void)hipStreamSynchronize(s);  // nothing in flight reads buf when it is freed
-    (void)hipFree(buf);
     return st;
 }
