@@ -320,7 +320,10 @@ typedef struct mf_plan_params {
  * elements at one node need pairwise different colors) and 255 CSR entries per row
  * (MF_ERR_ARG otherwise; the colored path has neither). The
  * build runs on up to 16 host threads (environment MF_PLAN_THREADS sets the count); the
- * plan does not depend on the count. */
+ * plan does not depend on the count. A small plan (default tile_lds_bytes, block_threads,
+ * max_tile_rows and id_chunks; coord given; too few default tiles for the GPU's CUs) holds
+ * a second schedule of smaller tiles, which mf_plan_assemble runs: same results. The
+ * calls that describe a plan and mf_plans_assemble use the default tiles. */
 int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nbNodes, int nnz,
                    const int *elemToNode, const int *row, const int *col,
                    const int *checkBounds, const double *coord,

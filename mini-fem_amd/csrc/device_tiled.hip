@@ -37,6 +37,7 @@ struct mf_plan {
     uint4 *task_rec = nullptr;
     int32_t *cb = nullptr;
     int32_t *isolated = nullptr;
+    mf_plan *alone = nullptr;  // the schedule of a launch of this plan alone, when it has one
 };
 
 namespace {
@@ -1037,6 +1038,7 @@ int upload_as(D **dst, const std::vector<S> &src)
 void free_plan(mf_plan *p)
 {
     if (!p) return;
+    free_plan(p->alone);
     void *ptrs[] = {p->tiles, p->tile_elems, p->tile_verts, p->tile_nodes, p->tile_rowinfo,
                     p->inc,   p->task_rec,   p->cb,
                     p->isolated};
@@ -1156,14 +1158,14 @@ int resolve_params(int op, const mf_plan_params *params, Resolved *r)
 
 int build_checked(mf::PlanHost &h, int op, int nE, int N, int nnz, const int *e2n,
                   const int *row, const int *col, const int *cb, const double *coord,
-                  const Resolved &r, int *lds64, int *lds32, int *back64 = nullptr,
+                  const Resolved &r, int parts, int *lds64, int *lds32, int *back64 = nullptr,
                   int *back32 = nullptr)
 {
     // the stage slot the tiles are sized by: a float-staged plan's FP64 layout may exceed
     // one CU's LDS, and that plan never launches in FP64
     const int slot = r.float_stage ? r.slot32 : r.slot64;
     int st = mf::build_plan(h, op, nE, N, nnz, e2n, row, col, cb, coord, r.budget, r.max_rows,
-                            slot, r.block, r.id_chunks);
+                            slot, r.block, r.id_chunks, parts);
     if (st != MF_OK) return st;
     st = mf::validate_plan(h, row, col, e2n, slot);
     if (st != MF_OK) return st;
@@ -1213,6 +1215,85 @@ bool valid_args(int op, int nE, int N, int nnz, const int *e2n, const int *row, 
            (nE == 0 || e2n) && row && (nnz == 0 || col);
 }
 
+using PlanGuard = std::unique_ptr<mf_plan, void (*)(mf_plan *)>;
+
+// Builds a schedule (parts as in build_plan) on the host.
+int make_schedule(PlanGuard &guard, mf::PlanHost &h, int parts, const Resolved &r, int op, int nE,
+                  int N, int nnz, const int *e2n, const int *row, const int *col,
+                  const int *checkBounds, const double *coord)
+{
+    int lds64 = 0, lds32 = 0, back64 = 0, back32 = 0;
+    const int st = build_checked(h, op, nE, N, nnz, e2n, row, col, checkBounds, coord, r, parts,
+                                 &lds64, &lds32, &back64, &back32);
+    if (st != MF_OK) return st;
+    guard.reset(new mf_plan);
+    mf_plan *p = guard.get();
+    p->op = op;
+    p->nE = nE;
+    p->N = N;
+    p->nnz = nnz;
+    p->dim = op == MF_OP_ELA ? 9 : 1;
+    p->ntiles = (int)h.tiles.size();
+    p->block = r.block;
+    p->lds_fp64 = lds64;
+    p->lds_mixed = lds32;
+    p->back_fp64 = back64;
+    p->back_mixed = back32;
+    p->n_isolated = (int)h.isolated.size();
+    p->float_stage = r.float_stage;
+    p->max_node = h.max_node;
+    p->max_elem = h.max_elem;
+    fill_stats(h, r.float_stage ? lds32 : lds64, r.block, p->stats);
+    return MF_OK;
+}
+
+// Puts a schedule on the GPU.
+int upload_schedule(mf_plan *p, const mf::PlanHost &h, const std::vector<int32_t> &cbHost)
+{
+    int rc = upload(&p->tiles, h.tiles);
+    if (rc == MF_OK) rc = upload(&p->tile_elems, h.tile_elems);
+    if (rc == MF_OK) rc = upload_as(&p->tile_verts, h.tile_verts);
+    if (rc == MF_OK) rc = upload(&p->tile_nodes, h.tile_nodes);
+    if (rc == MF_OK) rc = upload_as(&p->tile_rowinfo, h.tile_rowinfo);
+    if (rc == MF_OK) rc = upload(&p->inc, h.inc);
+    if (rc == MF_OK) rc = upload_as(&p->task_rec, h.task_rec);
+    if (rc == MF_OK) rc = upload(&p->isolated, h.isolated);
+    if (rc == MF_OK && !cbHost.empty()) rc = upload(&p->cb, cbHost);
+    if (rc == MF_OK)
+        rc = p->op == MF_OP_ELA ? prepare_all<MF_OP_ELA>(p) : prepare_all<MF_OP_LAP>(p);
+    return rc;
+}
+
+// How many tiles a launch of this plan alone is better cut into (0: as it is). The largest
+// tiles that fit have the least halo, but a tile is one workgroup's work from start to end,
+// and a CU holds one at a time: what they leave idle in the last round of tiles is better
+// spent on smaller ones. One tile per CU of the last round, so the number of rounds stays;
+// past kAloneRounds rounds the last one matters less than the time that the second schedule
+// takes to make (lap 38^3 20.7 and 17.8 us, but 33 and 45 ms), and a tile of fewer than
+// kAloneRows rows is no faster (its chain of loads and sums is the same). us, with the
+// default tiles and with these: ela 9^3 11.4 and 7.9, 16^3 11.7 and 8.3, 20^3 12.2 and 9.8,
+// 24^3 13.8 and 11.8, 28^3 21.7 and 18.4, 30^3 22.7 and 22.6; lap 9^3 6.6 and 5.5, 20^3 7.4
+// and 6.3, 30^3 12.0 and 11.1.
+// A launch of several plans keeps the default tiles: together they fill the CUs.
+constexpr int kAloneRounds = 2, kAloneRows = 12;
+
+int alone_parts(const mf::PlanHost &h, int *parts)
+{
+    int dev = 0, cus = 0;
+    *parts = 0;
+    const int T = (int)h.tiles.size(), rows = (int)h.tile_rowinfo.size();
+    if (T == 0) return MF_OK;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return MF_ERR_HIP;
+    cus = std::max(1, cus / kXcd) * kXcd;
+    const int rounds = (T + cus - 1) / cus;
+    if (rounds > kAloneRounds) return MF_OK;
+    const int p = std::min(rounds * cus, rows / kAloneRows);
+    if (10 * (int64_t)T < 9 * (int64_t)p) *parts = p;
+    return MF_OK;
+}
+
 }  // namespace
 
 extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nbNodes, int nnz,
@@ -1227,48 +1308,41 @@ extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nb
         Resolved r;
         int st = resolve_params(operatorID, params, &r);
         if (st != MF_OK) return st;
-        mf::PlanHost h;
-        int lds64 = 0, lds32 = 0, back64 = 0, back32 = 0;
-        st = build_checked(h, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col, checkBounds,
-                           coord, r, &lds64, &lds32, &back64, &back32);
+        mf::PlanHost h, ha;
+        PlanGuard guard(nullptr, free_plan), alone(nullptr, free_plan);
+        st = make_schedule(guard, h, 0, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
+                           checkBounds, coord);
+        if (st != MF_OK) return st;
+        // the second schedule, with the library's own tile sizes only
+        const bool sized = params && (params->tile_lds_bytes > 0 || params->max_tile_rows > 0 ||
+                                      params->block_threads > 0 || params->id_chunks > 1);
+        int parts = 0;
+        if (!sized && coord) st = alone_parts(h, &parts);
+        if (st == MF_OK && parts > 0)
+            st = make_schedule(alone, ha, parts, r, operatorID, nbElem, nbNodes, nnz, elemToNode,
+                               row, col, checkBounds, coord);
         if (st != MF_OK) return st;
 
-        // every host container is built before the first device allocation, and the plan
-        // is held by a guard until it is complete: an exception thrown here (bad_alloc)
-        // releases whatever device memory the plan already holds
+        // Every host container is built before the first device allocation, and the plan is
+        // held by a guard until it is complete: an exception thrown here (bad_alloc) releases
+        // whatever device memory the plan already holds. Both uploads come last, array by
+        // array: they leave the GPU awake for the first launch (lap 9^3: 23 us to its end,
+        // and 30 us after one large copy, or with host work between the uploads).
         std::vector<int32_t> cbHost;
         if (checkBounds && operatorID == MF_OP_ELA)
             cbHost.assign(checkBounds, checkBounds + (size_t)nbNodes * 3);
-        std::unique_ptr<mf_plan, void (*)(mf_plan *)> guard(new mf_plan, free_plan);
-        mf_plan *p = guard.get();
-        p->op = operatorID;
-        p->nE = nbElem;
-        p->N = nbNodes;
-        p->nnz = nnz;
-        p->dim = operatorID == MF_OP_ELA ? 9 : 1;
-        p->ntiles = (int)h.tiles.size();
-        p->block = r.block;
-        p->lds_fp64 = lds64;
-        p->lds_mixed = lds32;
-        p->back_fp64 = back64;
-        p->back_mixed = back32;
-        p->n_isolated = (int)h.isolated.size();
-        p->float_stage = r.float_stage;
-        p->max_node = h.max_node;
-        p->max_elem = h.max_elem;
-        int rc = upload(&p->tiles, h.tiles);
-        if (rc == MF_OK) rc = upload(&p->tile_elems, h.tile_elems);
-        if (rc == MF_OK) rc = upload_as(&p->tile_verts, h.tile_verts);
-        if (rc == MF_OK) rc = upload(&p->tile_nodes, h.tile_nodes);
-        if (rc == MF_OK) rc = upload_as(&p->tile_rowinfo, h.tile_rowinfo);
-        if (rc == MF_OK) rc = upload(&p->inc, h.inc);
-        if (rc == MF_OK) rc = upload_as(&p->task_rec, h.task_rec);
-        if (rc == MF_OK) rc = upload(&p->isolated, h.isolated);
-        if (rc == MF_OK && !cbHost.empty()) rc = upload(&p->cb, cbHost);
-        if (rc == MF_OK)
-            rc = operatorID == MF_OP_ELA ? prepare_all<MF_OP_ELA>(p) : prepare_all<MF_OP_LAP>(p);
-        if (rc != MF_OK) return rc;  // the guard frees the plan
-        fill_stats(h, r.float_stage ? lds32 : lds64, r.block, p->stats);
+        st = upload_schedule(guard.get(), h, cbHost);
+        if (st != MF_OK) return st;
+        if (alone && (int)ha.tiles.size() <= parts) {
+            // without room for it the plan does without
+            st = upload_schedule(alone.get(), ha, cbHost);
+            if (st == MF_OK)
+                guard->alone = alone.release();
+            else if (st == MF_ERR_NOMEM)
+                (void)hipGetLastError();
+            else
+                return st;
+        }
         *plan = guard.release();
         return MF_OK;
     });
@@ -1288,7 +1362,7 @@ extern "C" int mf_plan_host_stats(int operatorID, int nbElem, int nbNodes, int n
         mf::PlanHost h;
         int lds64 = 0, lds32 = 0;
         st = build_checked(h, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col, nullptr,
-                           coord, r, &lds64, &lds32);
+                           coord, r, 0, &lds64, &lds32);
         if (st != MF_OK) return st;
         fill_stats(h, r.float_stage ? lds32 : lds64, r.block, out);
         return MF_OK;
@@ -1350,6 +1424,7 @@ extern "C" int mf_plan_assemble(mf_plan *plan, const double *coord, const double
     if (!plan || !values || !prec || (plan->N > 0 && !coord)) return MF_ERR_ARG;
     if (precision == MF_PREC_FP64 && plan->float_stage) return MF_ERR_ARG;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    if (plan->alone) plan = plan->alone;
     const bool lap = plan->op == MF_OP_LAP;
     switch (precision) {
     case MF_PREC_FP64:

@@ -23,6 +23,10 @@ namespace {
 
 int plan_threads() { return host_threads(); }
 
+// Rows of a region whose halves, and tiles of a chunk, that are worth a thread: a tile takes
+// about 0.1 ms to find, 0.1 ms to write down and check, a thread 0.03 ms to start.
+constexpr int kSpawnRows = 768, kSpawnTiles = 4;
+
 // Map from non-negative ids to ints for the ids of one tile (a few hundred nodes, up to
 // ~1K elements), open addressing, cleared in O(1) by a generation counter. A map that
 // would pass half full reports it (insert returns -2) instead of degrading.
@@ -146,16 +150,9 @@ struct Partitioner {
                budget;
     }
 
-    // Recursive coordinate bisection along the longest axis. A region whose halves do
-    // not fit but whose thirds do is cut in three: tiles of a third rather than a quarter
-    // of it, i.e. fewer and larger tiles. The top levels run their halves on two threads.
-    // known: whether order[lo, hi) fits, when the caller has tested it (-1: not tested)
-    void rcb(int lo, int hi, FitScratch &s, std::vector<Leaf> &out, int depth, int known = -1)
+    // The axis along which order[lo, hi) is longest.
+    int widest(int lo, int hi) const
     {
-        if (hi - lo <= 1 || known == 1 || (known < 0 && fits(lo, hi, s))) {
-            if (hi > lo) out.emplace_back(lo, hi);
-            return;
-        }
         double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
         for (int i = lo; i < hi; i++)
             for (int d = 0; d < 3; d++) {
@@ -166,34 +163,110 @@ struct Partitioner {
         int ax = 0;
         for (int d = 1; d < 3; d++)
             if (mx[d] - mn[d] > mx[ax] - mn[ax]) ax = d;
-        const double *c = coord;
-        auto less = [c, ax](int a, int b) {
+        return ax;
+    }
+
+    struct ByCoord {
+        const double *c;
+        int ax;
+        bool operator()(int a, int b) const
+        {
             const double xa = c[(int64_t)a * 3 + ax], xb = c[(int64_t)b * 3 + ax];
             return xa < xb || (xa == xb && a < b);
-        };
-        // A cut near position p of order[a, b): the range is partitioned at p along the
-        // axis, then the cut moves to the widest coordinate gap within w of p. On a layered
-        // (e.g. jittered structured) mesh that gap lies between two layers of nodes, so a
-        // tile's faces are flat and its halo thin: at 100^3, 1.71 instead of 1.97 staged
-        // elements per element for lap tiles, which also grow larger under the same node cap.
-        auto cut = [&](int a, int b, int p, int w) {
-            std::nth_element(order.begin() + a, order.begin() + p, order.begin() + b, less);
-            const int l = std::max(a + 1, p - w), r = std::min(b - 1, p + w);
-            if (r - l < 2) return p;
-            std::nth_element(order.begin() + a, order.begin() + l, order.begin() + p, less);
-            std::nth_element(order.begin() + p, order.begin() + r, order.begin() + b, less);
-            std::sort(order.begin() + l, order.begin() + r, less);
-            double best = -1;
-            int bi = p;
-            for (int i = l + 1; i < r; i++) {
-                const double g = c[(int64_t)order[i] * 3 + ax] - c[(int64_t)order[i - 1] * 3 + ax];
-                if (g > best) {
-                    best = g;
-                    bi = i;
-                }
+        }
+    };
+    ByCoord by_coord(int ax) const { return ByCoord{coord, ax}; }
+
+    // A cut near position p of order[a, b): the range is partitioned at p along the axis,
+    // then the cut moves to the widest coordinate gap within w of p. On a layered (e.g.
+    // jittered structured) mesh that gap lies between two layers of nodes, so a tile's faces
+    // are flat and its halo thin: at 100^3, 1.71 instead of 1.97 staged elements per element
+    // for lap tiles, which also grow larger under the same node cap.
+    int cut_near(int a, int b, int p, int w, int ax)
+    {
+        const ByCoord less = by_coord(ax);
+        std::nth_element(order.begin() + a, order.begin() + p, order.begin() + b, less);
+        const int l = std::max(a + 1, p - w), r = std::min(b - 1, p + w);
+        if (r - l < 2) return p;
+        std::nth_element(order.begin() + a, order.begin() + l, order.begin() + p, less);
+        std::nth_element(order.begin() + p, order.begin() + r, order.begin() + b, less);
+        std::sort(order.begin() + l, order.begin() + r, less);
+        double best = -1;
+        int bi = p;
+        for (int i = l + 1; i < r; i++) {
+            const double g = coord[(int64_t)order[i] * 3 + ax] - coord[(int64_t)order[i - 1] * 3 + ax];
+            if (g > best) {
+                best = g;
+                bi = i;
             }
-            return bi;
-        };
+        }
+        return bi;
+    }
+
+    // order[lo, hi) in `parts` leaves of nearly equal size (a part that does not fit a tile
+    // is bisected further).
+    void split(int lo, int hi, int parts, FitScratch &s, std::vector<Leaf> &out, int depth = 0)
+    {
+        if (parts <= 1 || hi - lo <= 1) {
+            rcb(lo, hi, s, out, spawn_depth);
+            return;
+        }
+        const int left = parts / 2, p = lo + (int)((int64_t)(hi - lo) * left / parts);
+        const int mid = p > lo ? cut_near(lo, hi, p, (hi - lo) / parts / 4, widest(lo, hi)) : p;
+        two_halves(depth < spawn_depth && hi - lo > kSpawnRows, s, out,
+                   [&](FitScratch &t, std::vector<Leaf> &o) { split(lo, mid, left, t, o, depth + 1); },
+                   [&](FitScratch &t, std::vector<Leaf> &o) { split(mid, hi, parts - left, t, o, depth + 1); });
+    }
+
+    // f, then g, their leaves in that order; on two threads when asked to
+    template <class F, class G>
+    void two_halves(bool threads, FitScratch &s, std::vector<Leaf> &out, F f, G g)
+    {
+        if (!threads) {
+            f(s, out);
+            g(s, out);
+            return;
+        }
+        std::vector<Leaf> left, right;
+        bool spawned = false;
+        std::thread t;
+        try {
+            t = std::thread([&] {
+                try {
+                    FitScratch s2;
+                    f(s2, left);
+                } catch (...) {
+                    failed = 1;
+                }
+            });
+            spawned = true;
+        } catch (...) {
+        }
+        try {
+            if (!spawned) f(s, left);
+            g(s, right);
+        } catch (...) {  // join the other half before anything leaves this frame
+            failed = 1;
+        }
+        if (spawned) t.join();
+        if (failed) return;
+        out.insert(out.end(), left.begin(), left.end());
+        out.insert(out.end(), right.begin(), right.end());
+    }
+
+    // Recursive coordinate bisection along the longest axis. A region whose halves do
+    // not fit but whose thirds do is cut in three: tiles of a third rather than a quarter
+    // of it, i.e. fewer and larger tiles. The top levels run their halves on two threads.
+    // known: whether order[lo, hi) fits, when the caller has tested it (-1: not tested)
+    void rcb(int lo, int hi, FitScratch &s, std::vector<Leaf> &out, int depth, int known = -1)
+    {
+        if (hi - lo <= 1 || known == 1 || (known < 0 && fits(lo, hi, s))) {
+            if (hi > lo) out.emplace_back(lo, hi);
+            return;
+        }
+        const int ax = widest(lo, hi);
+        const auto less = by_coord(ax);
+        auto cut = [&](int a, int b, int p, int w) { return cut_near(a, b, p, w, ax); };
         // whether both halves of a cut at m fit; fl/fr: each half's result (-1: not tested)
         auto halves_fit = [&](int m, int &fl, int &fr) {
             fl = fits(lo, m, s) ? 1 : 0;
@@ -231,37 +304,9 @@ struct Partitioner {
             std::copy(saved.begin(), saved.end(), order.begin() + lo);  // back to the halves
         }
         // fl/fr hold for the halves of this cut: the recursion need not test them again
-        if (depth < spawn_depth && hi - lo > 4 * max_rows) {
-            std::vector<Leaf> left;
-            bool spawned = false;
-            std::thread t;
-            try {
-                t = std::thread([&] {
-                    try {
-                        FitScratch s2;
-                        rcb(lo, mid, s2, left, depth + 1, fl);
-                    } catch (...) {
-                        failed = 1;
-                    }
-                });
-                spawned = true;
-            } catch (...) {
-            }
-            std::vector<Leaf> right;
-            try {
-                if (!spawned) rcb(lo, mid, s, left, depth + 1, fl);
-                rcb(mid, hi, s, right, depth + 1, fr);
-            } catch (...) {  // join the other half before anything leaves this frame
-                failed = 1;
-            }
-            if (spawned) t.join();
-            if (failed) return;
-            out.insert(out.end(), left.begin(), left.end());
-            out.insert(out.end(), right.begin(), right.end());
-            return;
-        }
-        rcb(lo, mid, s, out, depth + 1, fl);
-        rcb(mid, hi, s, out, depth + 1, fr);
+        two_halves(depth < spawn_depth && hi - lo > kSpawnRows, s, out,
+                   [&](FitScratch &t, std::vector<Leaf> &o) { rcb(lo, mid, t, o, depth + 1, fl); },
+                   [&](FitScratch &t, std::vector<Leaf> &o) { rcb(mid, hi, t, o, depth + 1, fr); });
     }
 
     // Breadth-first order of the node graph (through shared elements), then greedy
@@ -511,7 +556,7 @@ struct Emitter {
 
 int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, const int *row,
                const int *col, const int *checkBounds, const double *coord, int lds_budget,
-               int max_rows, int slot_bytes, int block, int id_chunks)
+               int max_rows, int slot_bytes, int block, int id_chunks, int parts)
 {
     p = PlanHost{};
     p.op = op;
@@ -551,7 +596,8 @@ int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, cons
         // rowsAll is in ascending node id: contiguous ranges of it are id ranges
         FitScratch s;
         const int n = (int)rowsAll.size(), K = std::min(id_chunks, std::max(n, 1));
-        for (int k = 0; k < K; k++)
+        if (parts > 1) part.split(0, n, parts, s, leaves);
+        else for (int k = 0; k < K; k++)
             part.rcb((int)((int64_t)n * k / K), (int)((int64_t)n * (k + 1) / K), s, leaves, 0);
     } else {
         part.bfs_chunks(leaves);
@@ -566,7 +612,7 @@ int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, cons
 
     // the tiles in contiguous chunks, one per thread, then joined in order
     const Emitter em{ela, N, e2n, row, col, checkBounds, n2eI, n2eV, part.order, nodeTile, leaves};
-    const int nc = std::max(1, std::min(threads, T / 64));
+    const int nc = std::max(1, std::min(threads, T / kSpawnTiles));
     std::vector<TileChunk> chunks((size_t)nc);
     std::vector<std::thread> pool;
     pool.reserve((size_t)nc);
@@ -793,7 +839,7 @@ int validate_plan(const PlanHost &p, const int *row, const int *col, const int *
                            hit.data(), rowSeen.data()};
     // the tiles in contiguous chunks, one per thread; the first failure in any stops all
     const int T = (int)p.tiles.size();
-    const int nc = std::max(1, std::min(plan_threads(), T / 64));
+    const int nc = std::max(1, std::min(plan_threads(), T / kSpawnTiles));
     std::vector<int> status((size_t)nc, MF_OK);
     std::atomic<int> stop{0};
     auto run = [&](int c) {

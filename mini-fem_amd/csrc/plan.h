@@ -228,10 +228,11 @@ struct PlanHost {
 // for a workgroup of `block` threads hold. checkBounds (3N, ela) may be null.
 // id_chunks > 1: the rows are first cut into that many contiguous node-id ranges, and
 // each range is bisected on its own (tiles then hold rows of one id range, so the tiles
-// that run at the same time write nearby CSR rows).
+// that run at the same time write nearby CSR rows). parts > 1 (with coord): as many tiles of
+// nearly equal size, more only where one of them would not fit.
 int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, const int *row,
                const int *col, const int *checkBounds, const double *coord, int lds_budget,
-               int max_rows, int slot_bytes, int block, int id_chunks = 1);
+               int max_rows, int slot_bytes, int block, int id_chunks = 1, int parts = 0);
 
 // Checks every index the kernel will follow against the array it indexes, that every
 // CSR entry is written exactly once (diagonal, task or transpose) and that every task's

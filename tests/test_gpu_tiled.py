@@ -381,3 +381,33 @@ def test_plan_launched_from_two_host_threads(mf, orc, gpu):
     assert not errors, errors
     for v, p in outs:
         assert np.array_equal(v.numpy(), want_v) and np.array_equal(p.numpy(), want_p)
+
+
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("n", [2, 3, 5, 9, 14, 24, 28, 35])
+def test_small_plan_alone_equals_its_default_tiles(mf, gpu, op, n):
+    """A small plan has a second schedule for launches of its own, one tile per CU and round:
+    from one tile (2^3, 3^3) over one round (up to 24^3) and two (28^3) to the sizes that keep
+    the default tiles (35^3). Same values and prec as the default tiles (a plan whose tile
+    sizes the caller names has those alone), with a node outside every element, in every
+    mode, and in a launch of two plans, which takes the default tiles."""
+    print(f"[alone] op={op} n={n}", flush=True)
+    coord, e2n, code, nnz = mf.generate_cube(n, 0.25, 3, 7)
+    coord = np.concatenate([coord, [2.0, 2.0, 2.0]])
+    code = np.concatenate([code, [52]]).astype(np.int32)
+    mesh = mf.Mesh(coord, e2n, code, nnz + 1, op, coef=mf.generate_coef(op, e2n.size // 4, 5))
+    dm = gpu.DeviceMesh(mesh)
+    plan, sized = gpu.Plan(mesh), gpu.Plan(mesh, max_tile_rows=254)
+    assert plan.stats() == sized.stats()
+    for precision in (mf.PREC_FP64, mf.PREC_MIXED):
+        got = []
+        for run in (lambda: sized.assemble(dm.coord, dm.coef, dm.values, dm.prec, precision=precision),
+                    lambda: plan.assemble(dm.coord, dm.coef, dm.values, dm.prec, precision=precision),
+                    lambda: gpu.plans_assemble([(plan, dm.coord, dm.coef, dm.values, dm.prec)],
+                                               precision=precision)):
+            dm.values.fill(np.nan)
+            dm.prec.fill(np.nan)
+            run()
+            got.append((dm.values.numpy(), dm.prec.numpy()))
+        for v, p in got[1:]:
+            assert np.array_equal(v, got[0][0]) and np.array_equal(p, got[0][1], equal_nan=True)
