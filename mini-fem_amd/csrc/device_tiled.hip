@@ -1273,7 +1273,11 @@ int upload_schedule(mf_plan *p, const mf::PlanHost &h, const std::vector<int32_t
 // kAloneRows rows is no faster (its chain of loads and sums is the same). us, with the
 // default tiles and with these: ela 9^3 11.4 and 7.9, 16^3 11.7 and 8.3, 20^3 12.2 and 9.8,
 // 24^3 13.8 and 11.8, 28^3 21.7 and 18.4, 30^3 22.7 and 22.6; lap 9^3 6.6 and 5.5, 20^3 7.4
-// and 6.3, 30^3 12.0 and 11.1.
+// and 6.3, 30^3 12.0 and 11.1; Delaunay of 2,000 points ela 16.2 and 12.3, 10,000 lap 22.7 and
+// 20.4. Two rounds only where the rows' valences are alike: the longest incidence list is
+// the tile's longest chain whatever the tile's size, so two small tiles a CU then take as
+// long as two large ones, and more CUs wait for memory (Delaunay of 16,000 points, longest
+// list twice the mean: ela 43.8 and 53.3, lap of 18,000 26.5 and 32.8).
 // A launch of several plans keeps the default tiles: together they fill the CUs.
 constexpr int kAloneRounds = 2, kAloneRows = 12;
 
@@ -1289,6 +1293,13 @@ int alone_parts(const mf::PlanHost &h, int *parts)
     cus = std::max(1, cus / kXcd) * kXcd;
     const int rounds = (T + cus - 1) / cus;
     if (rounds > kAloneRounds) return MF_OK;
+    int64_t sum = 0, most = 0;
+    for (const mf::RowInfo &ri : h.tile_rowinfo) {
+        const int val = (ri.inc >> 16) & 0xFFFF;
+        sum += val;
+        most = std::max<int64_t>(most, val);
+    }
+    if (rounds > 1 && 2 * most * rows > 3 * sum) return MF_OK;
     const int p = std::min(rounds * cus, rows / kAloneRows);
     if (10 * (int64_t)T < 9 * (int64_t)p) *parts = p;
     return MF_OK;
