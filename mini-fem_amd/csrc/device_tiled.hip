@@ -534,35 +534,49 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
     } else {
         const int nwr = NC - nDB, wr = wave - nDB;
         if constexpr (ELA) {
-            // four rows per wave at a time, 16 lanes each. A row is 9 len doubles
-            // (~135) moved as 16-byte pieces, one 8-byte piece at the end of an
-            // odd-length row (8-byte aligned 16-byte stores are valid on gfx950; the
-            // LDS side reads two 8-byte words). A lane reads all its pieces of a pass
-            // (CP of them, 32 CP doubles per row and pass) before it stores any, so
-            // a row costs one LDS round trip, not one per piece.
-            constexpr int CP = 5;
-            const int g = lane >> 4, l16 = lane & 15;
-            for (int rr = wr * 4 + g; rr < R; rr += nwr * 4) {
-                const int4 ri = lri[rr];
+            // Four rows per wave at a time, 16 lanes each; a row is 9 len doubles (~135). The
+            // 128-byte lines that lie wholly in the row go out as non-temporal 16-byte
+            // stores, 8 lanes a line, and the ends of the row, whose lines the rows before and
+            // after it share, as plain 8-byte stores. Rows lie at any multiple of 8 bytes:
+            // as 16-byte pieces from the row's start, every piece straddles lines, and the
+            // cache writes the lines of rows in a random order out half full. Rows of 1080
+            // bytes, 1 GB, stores alone: in random order 330 us from the row's start, 345 by
+            // lines, 355 by lines and all of it non-temporal (half-full lines then go out at
+            // once), 181 like this; in order 180, 180, 250 and 162. ela 100^3 557 -> 484 us,
+            // 73^3 in node order 183 -> 173, 60^3 mixed 97.7 -> 87.9, 30^3 22.5 -> 20.0.
+            // A lane reads all its pieces (CP lines a 8 lanes) before it stores any, so a row
+            // costs one LDS round trip, and the next row's info is on its way meanwhile.
+            using Two = double __attribute__((ext_vector_type(2), aligned(8)));
+            constexpr int CP = 4;
+            const int g = lane >> 4, l16 = lane & 15, half = l16 >> 3, step = nwr * 4;
+            int4 next = lri[min(wr * 4 + g, R - 1)];
+            for (int rr = wr * 4 + g; rr < R; rr += step) {
+                const int4 ri = next;
+                next = lri[min(rr + step, R - 1)];
                 const int n = (ri.y & 0xFFFF) * 9;
                 const double *src = outv + (int64_t)ri.w * 9;
                 double *dst = jb.values + (int64_t)ri.x * 9;
-                for (int j0 = 2 * l16; j0 < n; j0 += 32 * CP) {
-                    double2 v[CP];
+                // the row: `head` doubles, `lines` whole lines, and what is left of it
+                const int head = min((int)(-(reinterpret_cast<uintptr_t>(dst) >> 3) & 15), n);
+                const int lines = (n - head) >> 4;
+                // the ends, up to 30 doubles: this lane's one or two
+                const int i0 = l16 < head ? l16 : l16 + 16 * lines, i1 = l16 + 16 + 16 * lines;
+                const double e0 = src[min(i0, n - 1)], e1 = src[min(i1, n - 1)];
+                const double *ls = src + head + 2 * l16;
+                double *ld = dst + head + 2 * l16;
+                Two v[CP];
 #pragma unroll
-                    for (int k = 0; k < CP; k++) {
-                        const int j = j0 + 32 * k;
-                        v[k] = make_double2(j < n ? src[j] : 0.0, j + 1 < n ? src[j + 1] : 0.0);
-                    }
+                for (int k = 0; k < CP; k++)
+                    if (half + 2 * k < lines) v[k] = Two{ls[32 * k], ls[32 * k + 1]};
 #pragma unroll
-                    for (int k = 0; k < CP; k++) {
-                        const int j = j0 + 32 * k;
-                        if (j + 1 < n)
-                            *reinterpret_cast<double2 *>(dst + j) = v[k];
-                        else if (j < n)
-                            dst[j] = v[k].x;
-                    }
-                }
+                for (int k = 0; k < CP; k++)
+                    if (half + 2 * k < lines)
+                        __builtin_nontemporal_store(v[k], reinterpret_cast<Two *>(ld + 32 * k));
+                for (int k = CP; half + 2 * k < lines; k++)  // rows of more than 15 blocks
+                    __builtin_nontemporal_store(Two{ls[32 * k], ls[32 * k + 1]},
+                                                reinterpret_cast<Two *>(ld + 32 * k));
+                if (i0 < n) dst[i0] = e0;
+                if (i1 < n) dst[i1] = e1;
             }
         } else {
             // four rows per wave, 16 lanes each
@@ -1277,7 +1291,7 @@ int upload_schedule(mf_plan *p, const mf::PlanHost &h, const std::vector<int32_t
 // 20.4. Two rounds only where the rows' valences are alike: the longest incidence list is
 // the tile's longest chain whatever the tile's size, so two small tiles a CU then take as
 // long as two large ones, and more CUs wait for memory (Delaunay of 16,000 points, longest
-// list twice the mean: ela 43.8 and 53.3, lap of 18,000 26.5 and 32.8).
+// list 84, mean 27: ela 43.8 and 53.3, lap of 18,000 26.5 and 32.8).
 // A launch of several plans keeps the default tiles: together they fill the CUs.
 constexpr int kAloneRounds = 2, kAloneRows = 12;
 

@@ -411,3 +411,30 @@ def test_small_plan_alone_equals_its_default_tiles(mf, gpu, op, n):
             got.append((dm.values.numpy(), dm.prec.numpy()))
         for v, p in got[1:]:
             assert np.array_equal(v, got[0][0]) and np.array_equal(p, got[0][1], equal_nan=True)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("offset", [0, 1, 8, 15])
+def test_rows_at_every_place_in_a_line(mf, orc, gpu, precision, offset):
+    """The ela copy-out stores a row's whole 128-byte lines and its two ends apart: rows of
+    7 to 25 blocks (up to 13 whole lines, past the 8 of one pass), starting at every multiple
+    of 8 bytes in a line, with the value array itself starting at a line, 8 bytes after one,
+    in the middle and 8 bytes before the end. Bit-exact, and nothing written around it."""
+    import bench
+    print(f"[line places] precision={precision} offset={offset}", flush=True)
+    coord, e2n, code, nnz = bench.delaunay_arrays(400, seed=9)
+    mesh = mf.Mesh(coord, e2n, code, nnz, mf.OP_ELA, coef=mf.generate_coef(1, e2n.size // 4, 5))
+    om = orc.OracleMesh(coord, e2n, code, nnz, mf.OP_ELA, coef=mf.generate_coef(1, e2n.size // 4, 5))
+    lengths = np.diff(mesh.row)
+    assert lengths.min() <= 8 and lengths.max() > 17
+    dm = gpu.DeviceMesh(mesh)
+    n = mesh.nnz * 9
+    room = gpu.DeviceArray.from_numpy(np.full(n + 48, -1.0))
+    start = (-(room.ptr // 8) % 16) + offset  # doubles from the buffer's start
+    values = gpu.DeviceView(room.ptr + 8 * start, n, np.float64, owner=room)
+    gpu.Plan(mesh, stage_precision=precision).assemble(dm.coord, dm.coef, values, dm.prec,
+                                                       precision=precision)
+    got = room.numpy()
+    ov = om.assemble(mixed=precision != 0)
+    assert np.array_equal(got[start:start + n], ov)
+    assert np.all(got[:start] == -1.0) and np.all(got[start + n:] == -1.0)
