@@ -310,41 +310,37 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
         __builtin_amdgcn_s_setprio(3);
         dri = dOn ? lri[r] : make_int4(0, 0, 0, 0);
         const int incOff = dri.z & 0xFFFF, val = dOn ? (dri.z >> 16) & 0xFFFF : 0;
-        // The row's incidence list, two entries per 32-bit word (lists are padded to a
-        // multiple of 4 entries), summed in order one pair at a time. Software
-        // pipelined: the LDS reads of the next pair are in flight while the current
-        // pair is summed; reads past the list repeat its last word and are never
-        // summed.
-        const uint32_t *lw = reinterpret_cast<const uint32_t *>(linc + incOff);
-        const int np = (val + 1) >> 1, lastw = val > 0 ? ((val + 3) >> 2) * 2 - 1 : 0;
-        auto word = [&](int q) { return lw[q < lastw ? q : lastw]; };
-        struct Pair {
-            T g[2][3];
-            T c[2][3];  // ela: lambda + 2 mu, lambda + mu, mu; lap: the product itself
-        };
-        auto fetch = [&](uint32_t w, Pair &P) {
+        if constexpr (ELA) {
+            // The row's incidence list, two entries per 32-bit word (lists are padded to a
+            // multiple of 4 entries), summed in order one pair at a time. Software
+            // pipelined: the LDS reads of the next pair are in flight while the current
+            // pair is summed; reads past the list repeat its last word and are never
+            // summed.
+            const uint32_t *lw = reinterpret_cast<const uint32_t *>(linc + incOff);
+            const int np = (val + 1) >> 1, lastw = val > 0 ? ((val + 3) >> 2) * 2 - 1 : 0;
+            auto word = [&](int q) { return lw[q < lastw ? q : lastw]; };
+            struct Pair {
+                T g[2][3];
+                T c[2][3];  // lambda + 2 mu, lambda + mu, mu
+            };
+            auto fetch = [&](uint32_t w, Pair &P) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const int e = u ? (int)(w >> 16) : (int)(w & 0xFFFF);
-                const T *sl = stage + (e >> 2) * S;
-                if constexpr (ELA) {
+                for (int u = 0; u < 2; u++) {
+                    const int e = u ? (int)(w >> 16) : (int)(w & 0xFFFF);
+                    const T *sl = stage + (e >> 2) * S;
                     ela_vertex(sl + 4 * (e & 3), P.g[u], P.c[u][0]);
                     const T2 c12 = *reinterpret_cast<const T2 *>(sl + 16);
                     P.c[u][1] = c12.x;
                     P.c[u][2] = c12.y;
-                } else {
-                    P.c[u][0] = sl[e & 3];
                 }
-            }
-        };
-        // ela_block(g, g) is exactly symmetric (g_d*g_e == g_e*g_d in IEEE): six
-        // sums hold the block bit for bit
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s4 = 0.0, s5 = 0.0, s8 = 0.0;
-        auto sum = [&](const Pair &P, int p) {
+            };
+            // ela_block(g, g) is exactly symmetric (g_d*g_e == g_e*g_d in IEEE): six
+            // sums hold the block bit for bit
+            double s0 = 0.0, s1 = 0.0, s2 = 0.0, s4 = 0.0, s5 = 0.0, s8 = 0.0;
+            auto sum = [&](const Pair &P, int p) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                if (2 * p + u >= val) break;
-                if constexpr (ELA) {
+                for (int u = 0; u < 2; u++) {
+                    if (2 * p + u >= val) break;
                     const T *g = P.g[u];
                     const T cd = P.c[u][0], co = P.c[u][1], cm = P.c[u][2];
                     const T p00 = g[0] * g[0], p11 = g[1] * g[1], p22 = g[2] * g[2];
@@ -354,31 +350,65 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
                     s4 += (double)(p00 * cm + p11 * cd + p22 * cm);
                     s5 += (double)(g[1] * g[2] * co);
                     s8 += (double)(p00 * cm + p11 * cm + p22 * cd);
-                } else {
-                    s0 += (double)P.c[u][0];
                 }
+            };
+            // LDS reads complete in issue order: each pair's list word is read before the
+            // previous pair's data, so waiting for the word leaves that data in flight
+            Pair A, B;
+            uint32_t wa = word(0), wb = word(1);
+            fetch(wa, A);  // pair 0
+            for (int p = 0; p < np; p += 2) {
+                wa = word(p + 2);
+                fetch(wb, B);  // pair p + 1
+                sum(A, p);
+                if (p + 1 >= np) break;
+                wb = word(p + 3);
+                fetch(wa, A);  // pair p + 2
+                sum(B, p + 1);
             }
-        };
-        // LDS reads complete in issue order: each pair's list word is read before the
-        // previous pair's data, so waiting for the word leaves that data in flight
-        Pair A, B;
-        uint32_t wa = word(0), wb = word(1);
-        fetch(wa, A);  // pair 0
-        for (int p = 0; p < np; p += 2) {
-            wa = word(p + 2);
-            fetch(wb, B);  // pair p + 1
-            sum(A, p);
-            if (p + 1 >= np) break;
-            wb = word(p + 3);
-            fetch(wa, A);  // pair p + 2
-            sum(B, p + 1);
-        }
-        if constexpr (ELA) {
             blk[0] = s0; blk[1] = s1; blk[2] = s2;
             blk[3] = s1; blk[4] = s4; blk[5] = s5;
             blk[6] = s2; blk[7] = s5; blk[8] = s8;
         } else {
-            blk[0] = s0;
+            // One read and one addition an entry: the reads' latency is what there is. Eight
+            // entries at a time (lists are padded to a multiple of 4, in 8-byte words), the
+            // next eight in flight meanwhile; reads past the list repeat its last word, and
+            // -0.0 stands for them in the sum, which it leaves as it is. Two at a time,
+            // this chain held barrier 2: lap 100^3 219 -> 217 us, 60^3 mixed 48.5 -> 42.6, 24^3
+            // 7.0 -> 6.5, 9^3 5.7 -> 5.2 (with the tasks' reads all at once as well).
+            const uint2 *lw = reinterpret_cast<const uint2 *>(linc + incOff);
+            const int lastw = val > 0 ? (val - 1) >> 2 : 0;
+            auto word = [&](int q) { return lw[q < lastw ? q : lastw]; };
+            auto fetch = [&](uint2 a, uint2 b, T (&x)[8]) {
+                const uint32_t w[4] = {a.x, a.y, b.x, b.y};
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int e = (int)((w[u >> 1] >> (16 * (u & 1))) & 0xFFFF);
+                    x[u] = stage[(e >> 2) * S + (e & 3)];
+                }
+            };
+            double s = 0.0;
+            auto sum = [&](const T (&x)[8], int j) {
+#pragma unroll
+                for (int u = 0; u < 8; u++) s += j + u < val ? (double)x[u] : -0.0;
+            };
+            T A[8], B[8];
+            uint2 a = word(0), b = word(1);
+            fetch(a, b, A);
+            a = word(2);
+            b = word(3);
+            for (int j = 0; j < val; j += 16) {
+                fetch(a, b, B);
+                a = word((j >> 2) + 4);
+                b = word((j >> 2) + 5);
+                sum(A, j);
+                if (j + 8 >= val) break;
+                fetch(a, b, A);
+                a = word((j >> 2) + 6);
+                b = word((j >> 2) + 7);
+                sum(B, j + 8);
+            }
+            blk[0] = s;
         }
         __builtin_amdgcn_s_setprio(0);
     } else {
@@ -456,6 +486,17 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
         } else if (rc.x != mf::kMaskRecord) {
             // up to kListLen contributions, padded with the zero slot TE
             const uint32_t w[3] = {rc.x, rc.y, rc.z};
+            if constexpr (!ELA) {  // one read each: all of them at once
+                T x[mf::kListLen];
+#pragma unroll
+                for (int u = 0; u < mf::kListLen; u++) {
+                    const int e = (int)((w[u >> 1] >> (16 * (u & 1))) & 0xFFFF);
+                    x[u] = stage[(e >> 4) * S + mf::lap_slot((e >> 2) & 3, e & 3)];
+                }
+#pragma unroll
+                for (int u = 0; u < mf::kListLen; u++) acc[0] += (double)x[u];
+                continue;
+            }
 #pragma unroll
             for (int u = 0; u < 3; u++) {
                 const int e0 = (int)(w[u] & 0xFFFF), e1 = (int)(w[u] >> 16);
@@ -543,7 +584,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
             // bytes, 1 GB, stores alone: in random order 330 us from the row's start, 345 by
             // lines, 355 by lines and all of it non-temporal (half-full lines then go out at
             // once), 181 like this; in order 180, 180, 250 and 162. ela 100^3 557 -> 484 us,
-            // 73^3 in node order 183 -> 173, 60^3 mixed 97.7 -> 87.9, 30^3 22.5 -> 20.0.
+            // 73^3 in node order 183 -> 175, 60^3 mixed 97.7 -> 88, 30^3 22.5 -> 20.1.
             // A lane reads all its pieces (CP lines a 8 lanes) before it stores any, so a row
             // costs one LDS round trip, and the next row's info is on its way meanwhile.
             using Two = double __attribute__((ext_vector_type(2), aligned(8)));
