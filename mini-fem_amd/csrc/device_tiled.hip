@@ -66,31 +66,64 @@ __device__ __forceinline__ void store_block9(double *dst, const double (&b)[9])
     dst[8] = b[8];
 }
 
-// ela stage slot: vertex v's group {gx, gy, gz, lambda+2mu} at sl + 4v (16-byte aligned).
-__device__ __forceinline__ void ela_vertex(const double *p, double (&g)[3], double &cd)
+// ela stage slot (mf::kStageEla64, kStageEla32): vertex v's gradient, and the element's
+// lambda + 2 mu, lambda + mu, mu. A double slot holds lambda and mu and the sums are taken
+// again by every reader; a float slot holds the sums, rounded from double.
+__device__ __forceinline__ void ela_vertex(const double *sl, int v, double (&g)[3])
 {
-    const double2 a = *reinterpret_cast<const double2 *>(p), b = *reinterpret_cast<const double2 *>(p + 2);
+    const double2 a = *reinterpret_cast<const double2 *>(sl + 2 * v);
     g[0] = a.x;
     g[1] = a.y;
-    g[2] = b.x;
-    cd = b.y;
+    g[2] = sl[8 + v];
 }
-__device__ __forceinline__ void ela_vertex(const float *p, float (&g)[3], float &cd)
+__device__ __forceinline__ void ela_vertex(const float *sl, int v, float (&g)[3])
 {
-    const float4 a = *reinterpret_cast<const float4 *>(p);
+    const float4 a = *reinterpret_cast<const float4 *>(sl + 4 * v);
     g[0] = a.x;
     g[1] = a.y;
     g[2] = a.z;
-    cd = a.w;
 }
-__device__ __forceinline__ void ela_vertex_store(double *p, const double (&g)[3], double cd)
+__device__ __forceinline__ void ela_coefs(const double *sl, int, double &cd, double &co, double &cm)
 {
-    *reinterpret_cast<double2 *>(p) = make_double2(g[0], g[1]);
-    *reinterpret_cast<double2 *>(p + 2) = make_double2(g[2], cd);
+    const double2 lm = *reinterpret_cast<const double2 *>(sl + 12);
+    cd = lm.x + 2.0 * lm.y;
+    co = lm.x + lm.y;
+    cm = lm.y;
 }
-__device__ __forceinline__ void ela_vertex_store(float *p, const double (&g)[3], double cd)
+__device__ __forceinline__ void ela_coefs(const float *sl, int v, float &cd, float &co, float &cm)
 {
-    *reinterpret_cast<float4 *>(p) = make_float4((float)g[0], (float)g[1], (float)g[2], (float)cd);
+    const float2 c = *reinterpret_cast<const float2 *>(sl + 16);
+    cd = sl[4 * v + 3];
+    co = c.x;
+    cm = c.y;
+}
+// An element's coefficients in the front (mf::front_coef_bytes), and its stage slot.
+__device__ __forceinline__ void ela_front(double *p, double lambda, double mu)
+{
+    *reinterpret_cast<double2 *>(p) = make_double2(lambda, mu);
+}
+__device__ __forceinline__ void ela_front(float *p, double lambda, double mu)
+{
+    p[0] = (float)(lambda + 2.0 * mu);
+    p[1] = (float)(lambda + mu);
+    p[2] = (float)mu;
+}
+__device__ __forceinline__ void ela_stage(double *sl, const double (&g)[4][3], const double *k)
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        *reinterpret_cast<double2 *>(sl + 2 * i) = make_double2(g[i][0], g[i][1]);
+    *reinterpret_cast<double2 *>(sl + 8) = make_double2(g[0][2], g[1][2]);
+    *reinterpret_cast<double2 *>(sl + 10) = make_double2(g[2][2], g[3][2]);
+    *reinterpret_cast<double2 *>(sl + 12) = *reinterpret_cast<const double2 *>(k);
+}
+__device__ __forceinline__ void ela_stage(float *sl, const double (&g)[4][3], const float *k)
+{
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        *reinterpret_cast<float4 *>(sl + 4 * i) =
+            make_float4((float)g[i][0], (float)g[i][1], (float)g[i][2], k[0]);
+    *reinterpret_cast<float2 *>(sl + 16) = make_float2(k[1], k[2]);
 }
 
 constexpr int kOpsAny = -1;  // operator per job, read from the job at run time
@@ -223,6 +256,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
     using T2 = typename Vec2<T>::type;
     constexpr int S = mf::stage_len(ELA, PREC == MF_PREC_FP64);
     constexpr int NA = ELA ? 9 : 1;
+    constexpr int KW = mf::front_coef_bytes(true, PREC == MF_PREC_FP64) / (int)sizeof(T);
     constexpr int NC = mf::compute_waves(BT), CT = NC * 64;
     constexpr int MAXE = mf::max_tile_elems(BT);
     constexpr int EA = (MAXE + CT - 1) / CT;  // A: elements per thread
@@ -257,11 +291,7 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
         T *sl = stage + t * S;
         if constexpr (ELA) {
             // src/assembly.cc:386-409 with per-element (lambda, mu)
-            const double2 lm = reinterpret_cast<const double2 *>(lds_raw + L.coef)[t];
-            const double cd = lm.x + 2.0 * lm.y, co = lm.x + lm.y, cm = lm.y;
-#pragma unroll
-            for (int i = 0; i < 4; i++) ela_vertex_store(sl + 4 * i, g[i], cd);
-            *reinterpret_cast<T2 *>(sl + 16) = T2{(T)co, (T)cm};
+            ela_stage(sl, g, reinterpret_cast<const T *>(lds_raw + L.coef) + t * KW);
         } else {
             // the element matrix, each product as the block sums take it
             const T kk = (T)reinterpret_cast<const double *>(lds_raw + L.coef)[t];
@@ -328,10 +358,8 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
                 for (int u = 0; u < 2; u++) {
                     const int e = u ? (int)(w >> 16) : (int)(w & 0xFFFF);
                     const T *sl = stage + (e >> 2) * S;
-                    ela_vertex(sl + 4 * (e & 3), P.g[u], P.c[u][0]);
-                    const T2 c12 = *reinterpret_cast<const T2 *>(sl + 16);
-                    P.c[u][1] = c12.x;
-                    P.c[u][2] = c12.y;
+                    ela_vertex(sl, e & 3, P.g[u]);
+                    ela_coefs(sl, e & 3, P.c[u][0], P.c[u][1], P.c[u][2]);
                 }
             };
             // ela_block(g, g) is exactly symmetric (g_d*g_e == g_e*g_d in IEEE): six
@@ -434,12 +462,9 @@ __device__ __forceinline__ void compute_tile(const mf::TileHdr &h, const TileJob
             for (int u = 0; u < 2; u++) {
                 const T *sl = stage + t[u] * S;
                 if constexpr (ELA) {
-                    T unused;
-                    ela_vertex(sl + 4 * a[u], ga[u], c0[u]);
-                    ela_vertex(sl + 4 * kk[u], gk[u], unused);
-                    const T2 c12 = *reinterpret_cast<const T2 *>(sl + 16);
-                    c1[u] = c12.x;
-                    c2[u] = c12.y;
+                    ela_vertex(sl, a[u], ga[u]);
+                    ela_vertex(sl, kk[u], gk[u]);
+                    ela_coefs(sl, a[u], c0[u], c1[u], c2[u]);
                 } else {
                     c0[u] = sl[mf::lap_slot(a[u], kk[u])];
                 }
@@ -828,11 +853,13 @@ __device__ __forceinline__ void tiled_body(const Jobs &J, int G, int f_node, int
                 if (i < hh.n_elem) lverts[i] = vert[r];
             }
             if (ela) {
-                double2 *lk = reinterpret_cast<double2 *>(lds_raw + L.coef);
+                using T = typename std::conditional<PREC == MF_PREC_FP64, double, float>::type;
+                constexpr int KW = mf::front_coef_bytes(true, PREC == MF_PREC_FP64) / (int)sizeof(T);
+                T *lk = reinterpret_cast<T *>(lds_raw + L.coef);
 #pragma unroll
                 for (int r = 0; r < EPT; r++) {
                     const int i = lt + r * LT;
-                    if (i < hh.n_elem) lk[i] = make_double2(hc ? k0[r] : 0.25, hc ? k1[r] : 1.0);
+                    if (i < hh.n_elem) ela_front(lk + i * KW, hc ? k0[r] : 0.25, hc ? k1[r] : 1.0);
                 }
             } else {
                 double *lk = reinterpret_cast<double *>(lds_raw + L.coef);
@@ -1219,24 +1246,37 @@ int build_checked(mf::PlanHost &h, int op, int nE, int N, int nnz, const int *e2
     // the stage slot the tiles are sized by: a float-staged plan's FP64 layout may exceed
     // one CU's LDS, and that plan never launches in FP64
     const int slot = r.float_stage ? r.slot32 : r.slot64;
-    int st = mf::build_plan(h, op, nE, N, nnz, e2n, row, col, cb, coord, r.budget, r.max_rows,
-                            slot, r.block, r.id_chunks, parts);
-    if (st != MF_OK) return st;
+    const bool ela = op == MF_OP_ELA;
+    int m64 = 0, m32 = 0, b64 = 0, b32 = 0;
+    auto measure = [&] {
+        m64 = m32 = b64 = b32 = 0;
+        for (const auto &t : h.tiles) {
+            // the front part (fixed offsets) is sized by the largest tile
+            const mf::TileLds L64 = mf::tile_lds_layout(ela, h.max_node, h.max_elem, t.n_elem,
+                                                        t.n_rows, t.n_inc, t.n_task, t.n_ent, r.slot64);
+            const mf::TileLds L32 = mf::tile_lds_layout(ela, h.max_node, h.max_elem, t.n_elem,
+                                                        t.n_rows, t.n_inc, t.n_task, t.n_ent, r.slot32);
+            m64 = std::max(m64, L64.total);
+            m32 = std::max(m32, L32.total);
+            b64 = std::max(b64, L64.total - L64.stage);
+            b32 = std::max(b32, L32.total - L32.stage);
+        }
+    };
+    // A tile is cut to the budget with a front of its own size: where the largest front and
+    // the largest back part belong to different tiles, the two may not fit a CU together, and
+    // the tiles are cut again to a budget smaller by what is too much.
+    int st = MF_OK, budget = r.budget;
+    for (int cut = 0;; cut++) {
+        st = mf::build_plan(h, op, nE, N, nnz, e2n, row, col, cb, coord, budget, r.max_rows, slot,
+                            r.block, r.id_chunks, parts);
+        if (st != MF_OK) return st;
+        measure();
+        const int over = (r.float_stage ? m32 : m64) + 16 - mf::kMaxLdsBytes;
+        if (over <= 0 || cut == 3 || budget - over < 4096) break;
+        budget -= over;
+    }
     st = mf::validate_plan(h, row, col, e2n, slot);
     if (st != MF_OK) return st;
-    int m64 = 0, m32 = 0, b64 = 0, b32 = 0;
-    for (const auto &t : h.tiles) {
-        // the front part (fixed offsets) is sized by the largest tile
-        const bool ela = op == MF_OP_ELA;
-        const mf::TileLds L64 = mf::tile_lds_layout(ela, h.max_node, h.max_elem, t.n_elem,
-                                                    t.n_rows, t.n_inc, t.n_task, t.n_ent, r.slot64);
-        const mf::TileLds L32 = mf::tile_lds_layout(ela, h.max_node, h.max_elem, t.n_elem,
-                                                    t.n_rows, t.n_inc, t.n_task, t.n_ent, r.slot32);
-        m64 = std::max(m64, L64.total);
-        m32 = std::max(m32, L32.total);
-        b64 = std::max(b64, L64.total - L64.stage);
-        b32 = std::max(b32, L32.total - L32.stage);
-    }
     if ((r.float_stage ? m32 : m64) + 16 > mf::kMaxLdsBytes)
         return MF_ERR_ARG;  // one row needs more than a CU has
     *lds64 = m64 + 16;
@@ -1512,11 +1552,11 @@ namespace {
 // LDS of a launch over several plans: the fixed front sized by their largest tiles with
 // ela's coefficient region (k_tiled_jobs keeps one front layout for both operators),
 // then the largest back part of any of their tiles.
-int jobs_lds(int f_node, int f_elem, int back)
+int jobs_lds(int f_node, int f_elem, int back, bool fp64)
 {
     const int verts = mf::align16(f_node * 24);
     const int coef = mf::align16(verts + (f_elem + 1) * 4);
-    return coef + mf::align16(f_elem * 16) + back + 16;
+    return coef + mf::align16(f_elem * mf::front_coef_bytes(true, fp64)) + back + 16;
 }
 
 // Persistent grid of k_tiled_jobs for `lds` bytes of LDS per workgroup: as many
@@ -1575,7 +1615,7 @@ int resolve_jobs(const mf_plan_job *jobs, int njobs, int precision, JobsLaunch &
         }
     }
     L.table.njobs = njobs;
-    L.lds = L.ntiles > 0 ? jobs_lds(L.f_node, L.f_elem, L.back) : 0;
+    L.lds = L.ntiles > 0 ? jobs_lds(L.f_node, L.f_elem, L.back, precision == MF_PREC_FP64) : 0;
     return L.lds > mf::kMaxLdsBytes ? MF_ERR_ARG : MF_OK;
 }
 

@@ -88,10 +88,16 @@ MF_HOST_DEVICE constexpr int max_tile_tasks(bool ela, int block)
 }
 
 // Element-stage slot of one tile element, in units of the stage type (double or float).
-//   ela: vertex v's {gx, gy, gz, lambda+2mu} at 4v, then {lambda+mu, mu} at 16: a vertex's
-//        gradient with the first coefficient is two 16-byte LDS reads in double, one in
-//        float. 144 bytes in double; 80 in float (16-byte multiples keep those reads
-//        aligned).
+//   ela, double: vertex v's gx, gy at 2v, its gz at 8 + v, {lambda, mu} at 12: 112 bytes, and
+//        40 (diagonal) or 64 to read for a contribution, which takes lambda + 2 mu and lambda +
+//        mu again itself. With those sums in the slot (144 bytes, {gx, gy, gz, lambda + 2 mu}
+//        a vertex; 48 and 80 to read) phase B moved a fifth more through LDS, which bounds
+//        it, and a tile held a fifth fewer elements: ela 100^3 486 -> 450 us, 73^3 in node order
+//        175 -> 162, 30^3 20.1 -> 18.7, Delaunay of 100,000 points 130 -> 119; 9^3, where
+//        the chain of a row counts, 8.0 -> 8.2.
+//   ela, float: vertex v's {gx, gy, gz, lambda+2mu} at 4v, then {lambda+mu, mu} at 16, each
+//        rounded from its value in double (float lambda and mu would not give them): a vertex
+//        is one 16-byte read. 80 bytes.
 //   lap: the element matrix k (g_i . g_j), i <= j: ten products, the four diagonal ones
 //        first (lap_slot). A contribution is then one 8-byte LDS read instead of the seven
 //        (two gradients and k) its product would take: 80 bytes in double, 40 in float. LDS
@@ -100,7 +106,7 @@ MF_HOST_DEVICE constexpr int max_tile_tasks(bool ela, int block)
 // Every length is an odd multiple of 16 (double) or 8 (float) bytes: consecutive elements
 // start in different LDS bank groups, so the per-element stage writes are conflict-free
 // and the gathers of scattered elements spread over all banks.
-constexpr int kStageEla64 = 18, kStageEla32 = 20;
+constexpr int kStageEla64 = 14, kStageEla32 = 20;
 constexpr int kStageLap = 10;
 // Place of the product of vertices a and k in a lap slot: (0,0) (1,1) (2,2) (3,3) (0,1)
 // (0,2) (0,3) (1,2) (1,3) (2,3), from a table of 16 nibbles.
@@ -113,6 +119,12 @@ MF_HOST_DEVICE constexpr int stage_len(bool ela, bool fp64)
     return ela ? (fp64 ? kStageEla64 : kStageEla32) : kStageLap;
 }
 
+// One element's coefficients in the front part of the LDS.
+//   ela, double: lambda, mu; ela, float: lambda + 2 mu, lambda + mu, mu, rounded from double,
+//   4 bytes less: the output image is what a tile's LDS holds besides in both, and tiles sized
+//   by the float stage stay the larger ones (100^3 12,860 and 13,008 tiles); lap: k in double.
+MF_HOST_DEVICE constexpr int front_coef_bytes(bool ela, bool fp64) { return ela ? (fp64 ? 16 : 12) : 8; }
+
 MF_HOST_DEVICE inline int align16(int x) { return (x + 15) & ~15; }
 
 // LDS of one tile, in two parts.
@@ -120,7 +132,7 @@ MF_HOST_DEVICE inline int align16(int x) { return (x + 15) & ~15; }
 // tile, f_node nodes and f_elem elements): the loader waves write the next tile's data
 // there while the compute waves still read the back part of the current tile.
 //   [node coordinates: f_node x 24 B] [element vertices: f_elem + 1 x 4 B]
-//   [raw coefficients: f_elem x 16 B (ela: lambda, mu) or 8 B (lap: k)]
+//   [coefficients: f_elem x front_coef_bytes]
 // The back part follows the tile's own sizes:
 //   [overlay: the element stage (n_elem + 1 slots, the last one all zero) during A and B,
 //             the output image (n_ent blocks of 9 doubles, ela, or 1, lap, in tile entry
@@ -131,7 +143,7 @@ struct TileLds {
     int coords, verts, coef, stage, rinfo, tasks, rnode, inc, total;
 };
 
-// front_ela: the front's coefficient region holds ela's 16 bytes per element (a launch
+// front_ela: the front's coefficient region holds ela's bytes per element (a launch
 // that mixes operators uses it for every tile); ela: the operator of the tile itself.
 MF_HOST_DEVICE inline TileLds tile_lds_layout(bool front_ela, bool ela, int f_node, int f_elem,
                                               int n_elem, int n_rows, int n_inc, int n_task,
@@ -141,7 +153,7 @@ MF_HOST_DEVICE inline TileLds tile_lds_layout(bool front_ela, bool ela, int f_no
     L.coords = 0;
     L.verts = align16(f_node * 24);
     L.coef = align16(L.verts + (f_elem + 1) * 4);
-    L.stage = L.coef + align16(f_elem * (front_ela ? 16 : 8));
+    L.stage = L.coef + align16(f_elem * front_coef_bytes(front_ela, slot_bytes == stage_len(ela, true) * 8));
     const int stage = (n_elem + 1) * slot_bytes, out = n_ent * (ela ? 72 : 8);
     L.rinfo = L.stage + align16(stage > out ? stage : out);
     L.tasks = L.rinfo + n_rows * 16;
