@@ -88,13 +88,12 @@ MF_HOST_DEVICE constexpr int max_tile_tasks(bool ela, int block)
 }
 
 // Element-stage slot of one tile element, in units of the stage type (double or float).
-//   ela, double: vertex v's gx, gy at 2v, its gz at 8 + v, {lambda, mu} at 12: 112 bytes, and
-//        40 (diagonal) or 64 to read for a contribution, which takes lambda + 2 mu and lambda +
-//        mu again itself. With those sums in the slot (144 bytes, {gx, gy, gz, lambda + 2 mu}
-//        a vertex; 48 and 80 to read) phase B moved a fifth more through LDS, which bounds
-//        it, and a tile held a fifth fewer elements: ela 100^3 486 -> 450 us, 73^3 in node order
-//        175 -> 162, 30^3 20.1 -> 18.7, Delaunay of 100,000 points 130 -> 119; 9^3, where
-//        the chain of a row counts, 8.0 -> 8.2.
+//   ela, double: vertex v's gx, gy at 2v, its gz at 8 + v, {lambda, mu} at 12: 112 bytes; a
+//        contribution takes lambda + 2 mu and lambda + mu itself. With those sums in the slot
+//        (144 bytes, {gx, gy, gz, lambda + 2 mu} a vertex) the stage bounded the tile, which
+//        held a fifth fewer elements: ela 100^3 486 -> 450 us, 73^3 in node order 175 -> 162,
+//        30^3 20.1 -> 18.7, Delaunay of 100,000 points 130 -> 119. (The tiles cut as before,
+//        with this slot: 492, so it is the larger tile; 9^3 8.0 -> 8.2.)
 //   ela, float: vertex v's {gx, gy, gz, lambda+2mu} at 4v, then {lambda+mu, mu} at 16, each
 //        rounded from its value in double (float lambda and mu would not give them): a vertex
 //        is one 16-byte read. 80 bytes.
