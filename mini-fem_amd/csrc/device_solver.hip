@@ -45,10 +45,14 @@ constexpr int kBT = 256;          // threads per workgroup
 // in the plan's order but 217 against 204 us in the shuffled one, 4 was slower in both
 constexpr int kGroup = 16;
 constexpr int kMaxGrid = 2048;    // workgroups of the reducing kernels (partials per sum)
-constexpr int kBatch = 8;         // iterations enqueued between two looks at the state
+// Iterations enqueued between two looks at the state: a look leaves the GPU idle for 30 us, an
+// iteration enqueued past the end costs 8, so 12, then a quarter of those so far, up to 32.
+// Eight each time, and these (us): lap 41^3, 20 iterations 544 and 508, 136 3143 and 2887; lap
+// 9^3, 46 iterations 889 and 778; ela 40^3, 304 iterations 11186 and 10327.
+constexpr int kBatch = 12, kMaxBatch = 32;
 
 // The iteration's scalars, on the device: the host enqueues iterations without waiting
-// for them and reads this after every kBatch. There are two: an iteration reads one and
+// for them and reads this after every batch. There are two: an iteration reads one and
 // k_direction writes the other, so no workgroup reads what another one writes. Once done is
 // set, every kernel of the iterations already enqueued returns at once.
 struct CgState {
@@ -532,11 +536,11 @@ static int pcg_core(bool ela, bool copied, int nbNodes, const int *row, const in
     else
         hipLaunchKernelGGL(k_start<false>, dim3(gNode), dim3(kBT), 0, s, b, q, prec, mask, nbNodes, r, z, part);
     direction(nullptr, cs);
-    // the iterations, enqueued kBatch at a time; k_direction counts each one and decides, as
+    // the iterations, enqueued a batch at a time; k_direction counts each one and decides, as
     // the loop condition would, whether another one runs
-    int done = 0, sent = 0;
+    int done = 0, sent = 0, batch = kBatch;
     do {
-        for (int k = 0; k < kBatch && sent < maxIter; k++, sent++) {
+        for (int k = 0; k < batch && sent < maxIter; k++, sent++) {
             const CgState *c = cs + (sent & 1);
             spmv(pm, p, q, c);
             if (ela)
@@ -554,6 +558,7 @@ static int pcg_core(bool ela, bool copied, int nbNodes, const int *row, const in
             return MF_ERR_HIP;
         }
         done = h.done;
+        batch = std::max(kBatch, std::min(sent / 4, kMaxBatch));
     } while (!done);
     if (iterations) *iterations = h.it;
     if (relResidual) *relResidual = std::sqrt(h.rr) / h.bnorm;
