@@ -1029,11 +1029,11 @@ __global__ void k_row_order(const mf::TileHdr *__restrict__ tiles, int ntiles,
 }
 
 // Write-only probe of the assembly's output stream. Mode 0: every tile row's CSR segment,
-// tiles dealt to XCDs and walked as k_tiled walks them, each segment written front to
-// back in 16-byte pieces (the copy-out of phase W); mode 1: the whole value array front to
-// back (the same bytes: the difference is what the row order costs in HBM); modes 2 and 3:
-// mode 0 split into the 128-byte lines a segment covers whole (2) and the partial lines
-// at its two ends, which it shares with the neighbouring rows (3).
+// tiles dealt to XCDs and walked as k_tiled walks them, each segment written as phase W
+// writes it (ela: whole lines non-temporal, its ends plain); mode 1: the whole value array
+// front to back (the same bytes: the difference is what the row order costs in HBM); modes 2
+// and 3: mode 0 split into the 128-byte lines a segment covers whole (2) and the partial
+// lines at its two ends, which it shares with the neighbouring rows (3).
 template <int D>
 __global__ void __launch_bounds__(1024)
     k_write_probe(const mf::TileHdr *__restrict__ tiles, int ntiles, int G,
@@ -1047,31 +1047,43 @@ __global__ void __launch_bounds__(1024)
         if (blockIdx.x == 0 && threadIdx.x == 0 && (total & 1)) values[total - 1] = 0.0;
         return;
     }
+    // 16 lanes a row, 64 rows at a time; the next tile's first rows are read before this
+    // one's are written, so that the probe times the writes and not these reads
+    using Two = double __attribute__((ext_vector_type(2), aligned(8)));
     const int per = (ntiles + kXcd - 1) / kXcd, xcd = blockIdx.x % kXcd;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
-    for (int slot = blockIdx.x / kXcd; slot < per && xcd * per + slot < ntiles; slot += G) {
-        const mf::TileHdr h = tiles[xcd * per + slot];
-        for (int r = wave; r < h.n_rows; r += nw) {
-            const int4 ri = rowinfo[h.rinfo_start + r];
-            const int64_t d0 = (int64_t)ri.x * D, d1 = d0 + (int64_t)(ri.y & 0xFFFF) * D;
-            if (mode == 0) {
-                for (int64_t j = d0 + 2 * lane; j < d1; j += 128) {
-                    if (j + 1 < d1) *reinterpret_cast<double2 *>(values + j) = make_double2(0.0, 0.0);
-                    else values[j] = 0.0;
-                }
-                continue;
-            }
-            // doubles [l0, l1) are the segment's whole 128-byte lines (16 doubles each)
-            const int64_t l0 = (d0 + 15) / 16 * 16, l1 = d1 / 16 * 16;
-            if (mode == 2) {
-                for (int64_t j = l0 + 2 * lane; j < l1; j += 128)
-                    *reinterpret_cast<double2 *>(values + j) = make_double2(0.0, 0.0);
-            } else {
-                const int64_t h1 = l0 < d1 ? l0 : d1, t0 = l1 > h1 ? l1 : h1;
-                for (int64_t j = d0 + lane; j < h1; j += 64) values[j] = 0.0;
-                for (int64_t j = t0 + lane; j < d1; j += 64) values[j] = 0.0;
-            }
+    const int last = min(per, ntiles - xcd * per), l16 = threadIdx.x & 15, r0 = threadIdx.x >> 4;
+    auto header = [&](int slot) { return tiles[xcd * per + min(slot, last - 1)]; };
+    auto info = [&](const mf::TileHdr &h, int r) { return rowinfo[h.rinfo_start + min(r, h.n_rows - 1)]; };
+    auto put = [&](const int4 &ri) {
+        double *dst = values + (int64_t)ri.x * D;
+        const int n = (ri.y & 0xFFFF) * D;
+        const int head = min((int)(-(reinterpret_cast<uintptr_t>(dst) >> 3) & 15), n);
+        const int tail = head + (n - head) / 16 * 16;  // whole 128-byte lines from head on
+        if (D == 9 && mode != 3)  // a loop of its own for each kind: one branch would lose `nt`
+            for (int j = head + 2 * l16; j < tail; j += 32)
+                __builtin_nontemporal_store(Two{0.0, 0.0}, reinterpret_cast<Two *>(dst + j));
+        if (D == 1 && mode != 3)
+            for (int j = head + 2 * l16; j < tail; j += 32)
+                *reinterpret_cast<Two *>(dst + j) = Two{0.0, 0.0};
+        if (mode != 2) {
+            if (l16 < head) dst[l16] = 0.0;
+            if (tail + l16 < n) dst[tail + l16] = 0.0;
         }
+    };
+    int slot = blockIdx.x / kXcd;
+    if (slot >= last) return;
+    mf::TileHdr h = header(slot), hn = header(slot + G);
+    int4 ri = info(h, r0), rj = info(h, r0 + 64);
+    for (; slot < last; slot += G) {
+        const int4 in = info(hn, r0), jn = info(hn, r0 + 64);
+        const mf::TileHdr hm = header(slot + 2 * G);
+        if (r0 < h.n_rows) put(ri);
+        if (r0 + 64 < h.n_rows) put(rj);
+        for (int r = r0 + 128; r < h.n_rows; r += 64) put(info(h, r));
+        h = hn;
+        hn = hm;
+        ri = in;
+        rj = jn;
     }
 }
 
