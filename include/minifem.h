@@ -307,7 +307,7 @@ typedef struct mf_plan_params {
     int stage_precision;  /* the precision mode the tiles are sized for. MF_PREC_FP64 (0,
                              default): the plan runs every mode. MF_PREC_MIXED or
                              MF_PREC_MIXED_F32COEF: tiles sized by the float stage, which
-                             holds twice the values per byte (ela 100^3: 18 % fewer tiles);
+                             takes a little less LDS (ela 100^3: 1 % fewer tiles);
                              the plan then runs the two mixed modes only, and FP64 launches
                              of it (mf_plan_assemble, mf_plans_assemble) return MF_ERR_ARG */
 } mf_plan_params;
@@ -320,8 +320,8 @@ typedef struct mf_plan_params {
  * elements at one node need pairwise different colors) and 255 CSR entries per row
  * (MF_ERR_ARG otherwise; the colored path has neither). The
  * build runs on up to 16 host threads (environment MF_PLAN_THREADS sets the count); the
- * plan does not depend on the count. A small plan (default tile_lds_bytes, block_threads,
- * max_tile_rows and id_chunks; coord given; too few default tiles for the GPU's CUs) holds
+ * plan does not depend on the count. A small plan (tile_lds_bytes, block_threads,
+ * max_tile_rows and id_chunks at their defaults; coord given; too few tiles for the GPU's CUs) holds
  * a second schedule of smaller tiles, which mf_plan_assemble runs: same results. The
  * calls that describe a plan and mf_plans_assemble use the default tiles. */
 int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nbNodes, int nnz,

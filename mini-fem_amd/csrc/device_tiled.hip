@@ -1379,7 +1379,7 @@ int upload_schedule(mf_plan *p, const mf::PlanHost &h, const std::vector<int32_t
 // takes to make (lap 38^3 20.7 and 17.8 us, but 33 and 45 ms), and a tile of fewer than
 // kAloneRows rows is no faster (its chain of loads and sums is the same). us, with the
 // default tiles and with these: ela 9^3 11.4 and 7.9, 16^3 11.7 and 8.3, 20^3 12.2 and 9.8,
-// 24^3 13.8 and 11.8, 28^3 21.7 and 18.4, 30^3 22.7 and 22.6; lap 9^3 6.6 and 5.5, 20^3 7.4
+// 24^3 13.8 and 11.8, 28^3 21.7 and 18.4, 30^3 22.7 and 21.5; lap 9^3 6.6 and 5.5, 20^3 7.4
 // and 6.3, 30^3 12.0 and 11.1; Delaunay of 2,000 points ela 16.2 and 12.3, 10,000 lap 22.7 and
 // 20.4. Two rounds only where the rows' valences are alike: the longest incidence list is
 // the tile's longest chain whatever the tile's size, so two small tiles a CU then take as
@@ -1432,8 +1432,10 @@ extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nb
                            checkBounds, coord);
         if (st != MF_OK) return st;
         // the second schedule, with the library's own tile sizes only
-        const bool sized = params && (params->tile_lds_bytes > 0 || params->max_tile_rows > 0 ||
-                                      params->block_threads > 0 || params->id_chunks > 1);
+        Resolved own;
+        (void)resolve_params(operatorID, nullptr, &own);
+        const bool sized = r.budget != own.budget || r.block != own.block ||
+                           r.max_rows != own.max_rows || r.id_chunks != own.id_chunks;
         int parts = 0;
         if (!sized && coord) st = alone_parts(h, &parts);
         if (st == MF_OK && parts > 0)

@@ -21,7 +21,7 @@
 //      - a diagonal block (the whole incidence list) is one lane;
 //   O) put every block of the tile's rows into an LDS output image of those rows' CSR
 //      segments, laid over the element stage;
-//   W) copy the image row by row to the CSR value array in consecutive 16-byte pieces,
+//   W) copy the image row by row to the CSR value array, whole 128-byte lines non-temporal,
 //      while the diagonal lanes invert their blocks into the block-Jacobi prec
 //      (prec_init + prec_inversion fused). Meanwhile the loader waves write the next
 //      tile's coordinates, coefficients and element vertices into LDS.

@@ -397,7 +397,7 @@ def test_small_plan_alone_equals_its_default_tiles(mf, gpu, op, n):
     code = np.concatenate([code, [52]]).astype(np.int32)
     mesh = mf.Mesh(coord, e2n, code, nnz + 1, op, coef=mf.generate_coef(op, e2n.size // 4, 5))
     dm = gpu.DeviceMesh(mesh)
-    plan, sized = gpu.Plan(mesh), gpu.Plan(mesh, max_tile_rows=254)
+    plan, sized = gpu.Plan(mesh), gpu.Plan(mesh, max_tile_rows=253)
     assert plan.stats() == sized.stats()
     for precision in (mf.PREC_FP64, mf.PREC_MIXED):
         got = []
