@@ -111,18 +111,15 @@ struct RowsCtl {
     unsigned found[kRowsGridMax];  // table entries of each rows workgroup that are elements
 };
 
-// Whether the rows left a call of nE elements to what follows them: they found something odd, a
-// node id past the table's `rows`, or not 4 table entries per element. Called by a whole
-// workgroup of BT threads; s: one word of LDS per thread.
+// Whether the rows left a call of nE elements to what follows them: they found something odd,
+// or not 4 table entries per element. Called by a whole workgroup of BT threads; s: one word of
+// LDS per thread.
 template <int BT>
-__device__ bool rows_verdict(const RowsCtl *ctl, int tables, int groups, int rows, int nE,
-                             unsigned long long *s)
+__device__ bool rows_verdict(const RowsCtl *ctl, int groups, int nE, unsigned long long *s)
 {
     unsigned long long n = 0;
-    bool past = false;
     for (int w = threadIdx.x; w < groups; w += BT) n += ctl->found[w];
-    for (int w = threadIdx.x; w < tables; w += BT) past |= ctl->top[w] > rows;
-    s[threadIdx.x] = past ? 1ull << 50 : n;
+    s[threadIdx.x] = n;
     __syncthreads();
     for (int w = BT / 2; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
@@ -160,10 +157,10 @@ __global__ void __launch_bounds__(1024)
                             const double *__restrict__ coef, double *values,
                             const int *__restrict__ row, const int *__restrict__ col,
                             const int4 *__restrict__ e2n, const int *__restrict__ e2e, int64_t nv,
-                            const RowsCtl *__restrict__ ctl, int tables, int groups, int rows)
+                            const RowsCtl *__restrict__ ctl, int groups)
 {
     __shared__ unsigned long long s[1024];
-    if (!rows_verdict<1024>(ctl, tables, groups, rows, co.off[co.n], s)) return;
+    if (!rows_verdict<1024>(ctl, groups, co.off[co.n], s)) return;
     for (int64_t z = threadIdx.x; z < nv; z += 1024) values[z] = 0.0;
     for (int c = 0; c < co.n; c++) {
         __syncthreads();
@@ -184,12 +181,18 @@ __global__ void __launch_bounds__(1024)
 // only if it names an element of its color that holds the node, and the slots that elements
 // own are always written.
 //
-// The call does not say how many nodes there are; the table holds nnz / 4 of them, which a
-// pattern with the elements' own couplings leaves (4 entries for each node of an element).
+// The call does not say how many nodes there are, and a part of a mesh may keep the ids of the
+// whole. The first nnz / 8 nodes (rows have 15 entries in the mean, so those are all unless ids
+// are left out) have the line of their id in the table; a node past them has the line, after
+// those, of a quarter of its row's start. The row of a node of an element has 4 entries or more
+// (the element's own couplings), so no two such nodes share a line, and nnz / 4 lines hold them
+// whatever the ids. Without those lines the launch after the rows took such a call: ela 40^3
+// with ids eight times as far 62,000 us, so 337. All nodes by their rows' starts: lap 100^3
+// 1,560 -> 1,889, ela 60^3 353 -> 369.
 // What the rows cannot do is left to the launches after them, which otherwise return at once:
 // an elemToEdge entry outside its node's row or a diagonal entry that not all of the node's
-// elements share (k_entry_*), node ids past the table, and elements of one color that share a
-// node or elements that repeat one (k_assemble_colors_one).
+// elements share (k_entry_*), and, without elemToEdge, elements of one color that share a node,
+// elements that repeat one and rows of fewer entries (k_assemble_colors_one).
 //
 // ela 60^3 1,830 -> 416 us, lap 31^3 with elemToEdge 148 -> 53 (the two prec
 // calls included); ela 60^3: k_row_table 63 us, k_assemble_rows 293.
@@ -210,9 +213,21 @@ __device__ __forceinline__ int color_of(const ColorOffsets &co, int e0, int e, i
     return c;
 }
 
+// The lines of the table of a call of nnz entries: by id, then by the row's start.
+__host__ __device__ constexpr int direct_lines(int nnz) { return nnz / 8 + 1; }
+__host__ __device__ constexpr int table_lines(int nnz) { return direct_lines(nnz) + nnz / 4 + 1; }
+
+// The line of node i (0-based); -1 where its row starts outside the entries.
+__device__ __forceinline__ int line_of(int i, const int *__restrict__ row, int nnz)
+{
+    if (i < direct_lines(nnz)) return i;
+    const int start = row[i];
+    return start >= 0 && start <= nnz ? direct_lines(nnz) + (start >> 2) : -1;
+}
+
 __global__ void __launch_bounds__(kBlock)
-    k_row_table(ColorOffsets co, const int4 *__restrict__ e2n, int nE, int cap, int width,
-                int *__restrict__ table, RowsCtl *__restrict__ ctl)
+    k_row_table(ColorOffsets co, const int4 *__restrict__ e2n, const int *__restrict__ row, int nE,
+                int nnz, int width, int *__restrict__ table, RowsCtl *__restrict__ ctl)
 {
     __shared__ int smax[kBlock / 64];
     int top = 0;
@@ -226,8 +241,10 @@ __global__ void __launch_bounds__(kBlock)
         const int v[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int k = 0; k < 4; k++) {
+            const int i = v[k] - 1;
             top = top > v[k] ? top : v[k];
-            if (v[k] >= 1 && v[k] <= cap) table[(int64_t)(v[k] - 1) * width + c] = e;
+            const int line = i < 0 ? -1 : line_of(i, row, nnz);
+            if (line >= 0) table[(int64_t)line * width + c] = e;
         }
     }
 #pragma unroll
@@ -259,7 +276,7 @@ __global__ void __launch_bounds__(64)
                     const double *__restrict__ coef, double *__restrict__ values,
                     const int *__restrict__ row, const int *__restrict__ col,
                     const int4 *__restrict__ e2n, const int *__restrict__ e2e, int nnz,
-                    const int *__restrict__ table, RowsCtl *__restrict__ ctl, int tables, int rows)
+                    const int *__restrict__ table, RowsCtl *__restrict__ ctl, int tables)
 {
     using T = typename std::conditional<PREC == MF_PREC_FP64, double, float>::type;
     constexpr bool ELA = OP == MF_OP_ELA;
@@ -291,7 +308,7 @@ __global__ void __launch_bounds__(64)
         const int t = __shfl_xor(N, o);
         N = N > t ? N : t;
     }
-    N = __builtin_amdgcn_readfirstlane(N < rows ? N : rows);
+    N = __builtin_amdgcn_readfirstlane(N);
     const int quads = (N + 3) / 4;
     // the XCD of a workgroup walks its eighth of the rows: neighbouring rows share elements
     const int per = (quads + 7) / 8, xcd = blockIdx.x & 7, step = gridDim.x >> 3;
@@ -306,9 +323,9 @@ __global__ void __launch_bounds__(64)
         r1 = row[ic + 1];
     };
     auto slots = [&](int s, int (&e)[KC]) {
-        const int i = row_of(s), ic = i < N ? i : 0;
+        const int i = row_of(s), q = line_of(i < N ? i : 0, row, nnz), line = q < 0 ? 0 : q;
 #pragma unroll
-        for (int k = 0; k < KC; k++) e[k] = table[(int64_t)ic * (16 * KC) + l + 16 * k];
+        for (int k = 0; k < KC; k++) e[k] = table[(int64_t)line * (16 * KC) + l + 16 * k];
     };
     auto elements = [&](const int (&e)[KC], int4 (&q)[KC]) {
 #pragma unroll
@@ -591,11 +608,10 @@ __global__ void __launch_bounds__(64)
 // each color. Nothing is assumed of the positions but that.
 __global__ void __launch_bounds__(kBlock)
     k_entry_table(ColorOffsets co, const int *__restrict__ e2e, int nE, int nnz, int width,
-                  uint32_t *__restrict__ table, RowsCtl *__restrict__ ctl, int tables, int groups,
-                  int rows)
+                  uint32_t *__restrict__ table, RowsCtl *__restrict__ ctl, int groups)
 {
     __shared__ unsigned long long s[kBlock];
-    const bool left = rows_verdict<kBlock>(ctl, tables, groups, rows, nE, s);
+    const bool left = rows_verdict<kBlock>(ctl, groups, nE, s);
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->left = left;
     if (!left) return;
     const int lane = threadIdx.x & 63;
@@ -755,19 +771,19 @@ int launch_colors(const double *coord, const double *coef, double *values, const
 template <int OP, int PREC, bool EDGES>
 void launch_rows_width(int kc, const ColorOffsets &co, const double *coord, const double *coef,
                        double *values, const int *row, const int *col, const int4 *e2n,
-                       const int *e2e, int nnz, const int *table, RowsCtl *ctl, int tables, int rows,
+                       const int *e2e, int nnz, const int *table, RowsCtl *ctl, int tables,
                        int groups, hipStream_t s)
 {
     const dim3 g((unsigned)groups), b(64);
     if (kc == 2)
         hipLaunchKernelGGL((k_assemble_rows<OP, PREC, EDGES, 2>), g, b, 0, s, co, coord, coef,
-                           values, row, col, e2n, e2e, nnz, table, ctl, tables, rows);
+                           values, row, col, e2n, e2e, nnz, table, ctl, tables);
     else if (kc == 4)
         hipLaunchKernelGGL((k_assemble_rows<OP, PREC, EDGES, 4>), g, b, 0, s, co, coord, coef,
-                           values, row, col, e2n, e2e, nnz, table, ctl, tables, rows);
+                           values, row, col, e2n, e2e, nnz, table, ctl, tables);
     else
         hipLaunchKernelGGL((k_assemble_rows<OP, PREC, EDGES, 8>), g, b, 0, s, co, coord, coef,
-                           values, row, col, e2n, e2e, nnz, table, ctl, tables, rows);
+                           values, row, col, e2n, e2e, nnz, table, ctl, tables);
 }
 
 // The row-by-row assembly; false when it does not apply (the caller then runs the colors): a
@@ -792,7 +808,6 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
     co.n = nbColors;
     std::memcpy(co.off, colorToElem, (size_t)(nbColors + 1) * sizeof(int));
     const int kc = nbColors <= 32 ? 2 : nbColors <= 64 ? 4 : 8, width = 16 * kc;
-    const int rows = nnz / 4 + 1;
     const int tables = (int)std::min<unsigned>(kTableGrid, grid_for(nbElem));
     // as many workgroups as a CU's LDS holds (ela, FP64: 8; else 16 cover the latency), at
     // most one per four rows of 4 entries, a multiple of 8 (one share per XCD)
@@ -800,7 +815,7 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
     static_assert(256 * kPerCu <= kRowsGridMax, "one slot per workgroup");
     const int groups = (int)std::min<int64_t>(256 * kPerCu, ((int64_t)nnz / 16 + 8) / 8 * 8);
     const size_t head = (sizeof(RowsCtl) + 255) / 256 * 256;
-    const size_t bytes = head + (size_t)(e2e ? nnz : rows) * width * sizeof(int);
+    const size_t bytes = head + (size_t)std::max(e2e ? nnz : 0, table_lines(nnz)) * width * sizeof(int);
     unsigned char *buf = nullptr;
     if (hipMallocFromPoolAsync(reinterpret_cast<void **>(&buf), bytes, pool, s) != hipSuccess) {
         (void)hipGetLastError();
@@ -809,24 +824,25 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
     RowsCtl *ctl = reinterpret_cast<RowsCtl *>(buf);
     int *table = reinterpret_cast<int *>(buf + head);
     const int4 *en = reinterpret_cast<const int4 *>(e2n);
-    hipLaunchKernelGGL(k_row_table, dim3((unsigned)tables), dim3(kBlock), 0, s, co, en, nbElem, rows,
-                       width, table, ctl);
+    hipLaunchKernelGGL(k_row_table, dim3((unsigned)tables), dim3(kBlock), 0, s, co, en, row, nbElem,
+                       nnz, width, table, ctl);
     if (e2e) {
         launch_rows_width<OP, PREC, true>(kc, co, coord, coef, values, row, col, en, e2e, nnz, table,
-                                          ctl, tables, rows, groups, s);
+                                          ctl, tables, groups, s);
         // any table of positions may be: these return at once unless the rows left the call
         uint32_t *entries = reinterpret_cast<uint32_t *>(table);
         hipLaunchKernelGGL(k_entry_table, dim3(256), dim3(kBlock), 0, s, co, e2e, nbElem, nnz, width,
-                           entries, ctl, tables, groups, rows);
+                           entries, ctl, groups);
         hipLaunchKernelGGL((k_entry_sum<OP, PREC>), dim3(1024), dim3(kBlock), 0, s, co, coord, coef,
                            values, en, e2e, nnz, width, entries, ctl);
     } else {
         launch_rows_width<OP, PREC, false>(kc, co, coord, coef, values, row, col, en, e2e, nnz, table,
-                                           ctl, tables, rows, groups, s);
-        // left: a numbering most of whose rows are empty, or an invalid coloring
+                                           ctl, tables, groups, s);
+        // left: rows shorter than an element's couplings, a vertex that stands twice in an
+        // element, or an invalid coloring
         hipLaunchKernelGGL((k_assemble_colors_one<OP, PREC>), dim3(1), dim3(1024), 0, s, co, coord,
                            coef, values, row, col, en, e2e,
-                           (int64_t)nnz * (OP == MF_OP_ELA ? 9 : 1), ctl, tables, groups, rows);
+                           (int64_t)nnz * (OP == MF_OP_ELA ? 9 : 1), ctl, groups);
     }
     const bool ok = hipGetLastError() == hipSuccess;
     *status = hipFreeAsync(buf, s) == hipSuccess && ok ? MF_OK : MF_ERR_HIP;

@@ -134,3 +134,58 @@ def test_rows_odd_edges(mf, gpu, op, n):
     for a, b in zip(m.row[:-1], m.row[1:]):
         perm[a:b] = a + rng.permutation(b - a)
     same(both(mf, gpu, m, perm[e2e]), "permuted rows")
+
+
+def times(mf, gpu, mesh, row, col, e2n):
+    """ms of (row by row, color by color), without elemToEdge, the least of five calls each."""
+    D = gpu.DeviceArray.from_numpy
+    coord, k, row, col, e2n = D(mesh.coord), D(mesh.coef), D(row), D(col), D(e2n)
+    values, stream = gpu.DeviceArray(mesh.nnz * mesh.dim, np.float64), gpu.Stream()
+
+    def call(s):
+        gpu.assembly(coord, values, row, col, e2n, None, mesh.nbElem, mesh.nnz, mesh.dim,
+                     mesh.operatorID, mesh.colorToElem, coef=k, stream=s)
+
+    graph, a, b, got = gpu.Graph(stream, call), gpu.Event(), gpu.Event(), []
+    for run in (lambda: call(stream), lambda: graph.launch(stream)):
+        ms = []
+        for _ in range(6):
+            a.record(stream)
+            run()
+            b.record(stream)
+            stream.sync()
+            ms.append(a.elapsed_ms(b))
+        got.append(min(ms[1:]))
+    return got
+
+
+def wide_ids(mf, mesh, far, seed=4):
+    """The mesh as a part that keeps the ids of a whole `far` times as large (in no order):
+    (coord, row, col, elemToNode)."""
+    N = mesh.nbNodes
+    ids = np.random.default_rng(seed).permutation(far * N)[:N]
+    order = np.argsort(ids)  # the part's nodes by their new ids
+    lengths = np.zeros(far * N, np.int64)
+    lengths[ids] = np.diff(mesh.row)
+    row = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    col = np.concatenate([ids[mesh.col[mesh.row[i]:mesh.row[i + 1]] - 1] + 1 for i in order])
+    coord = np.zeros((far * N, 3))
+    coord[ids] = mesh.coord.reshape(-1, 3)
+    return coord.ravel(), row, col.astype(np.int32), (ids[mesh.elemToNode - 1] + 1).astype(np.int32)
+
+
+@pytest.mark.parametrize("op,far", [(0, 5), (1, 5), (1, 40)])
+def test_rows_of_a_part_that_keeps_global_ids(mf, gpu, op, far):
+    """Ids far past a quarter of the entries are valid input: they get the same values as from
+    one launch per color, and not more slowly."""
+    print(f"[rows wide] op={op} far={far}", flush=True)
+    coord, e2n, code, nnz = mf.generate_cube(30, 0.25, 3, 11)
+    m = mf.Mesh(coord, e2n, code, nnz, op, coef=mf.generate_coef(op, e2n.size // 4, 9))
+    wide = mf.Mesh.__new__(mf.Mesh)
+    wide.__dict__.update(m.__dict__)
+    wide.coord, row, col, e2n = wide_ids(mf, m, far)
+    assert e2n.max() > m.nnz // 4 + 1
+    same(both(mf, gpu, wide, row=row, col=col, e2n=e2n), f"ids {far}")
+    rows, colors = times(mf, gpu, wide, row=row, col=col, e2n=e2n)
+    print(f"  rows {rows:.3f} ms, colors {colors:.3f} ms", flush=True)
+    assert rows < 2 * colors
