@@ -216,7 +216,8 @@ int mf_gather_probe(double *dst, const double *src, const int64_t *idx, int64_t 
  * entry from zero and in color order, the blocks of elements [colorToElem[c],
  * colorToElem[c+1]), c = 0, 1, ..., of the color-permuted elemToNode (elements of one color
  * share no node). The call takes stream-ordered workspace from a pool of the library's own,
- * about 1.5 bytes per CSR entry and color (4 with elemToEdge); under stream capture, or where
+ * 1.5 bytes per CSR entry and color (their number rounded up to 32, 64 or 128), with
+ * elemToEdge 4 bytes per CSR entry more; under stream capture, or where
  * there is no memory for it, it runs one launch per color instead. elemToEdge (device, 16
  * per element) gives the scatter positions; NULL selects the reference's default row search
  * (src/assembly.cc:415-421). colorToElem is a HOST array of nbColors+1 offsets (the

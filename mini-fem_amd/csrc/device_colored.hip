@@ -4,7 +4,9 @@
 //   prec_inversion()  -> mf_prec_inversion
 //   compute_double_norm() -> mf_norm
 // The assembly goes row by row (k_assemble_rows): the per-entry summation order is the color
-// order, i.e. the reference COLORING build's element order. Under stream capture, without
+// order, i.e. the reference COLORING build's element order. What the rows cannot do goes on, in
+// the same order, in launches after them that ordinarily return at once (k_entry_* with
+// elemToEdge, else k_assemble_left). Under stream capture, without
 // memory for its workspace and for patterns thinner than the elements' couplings it is one
 // launch per color with 16 lanes per element (one per element block): elements of one color
 // share no node, so their scatter-adds never touch the same CSR entry and each pass is
@@ -106,9 +108,9 @@ struct ColorOffsets {
 constexpr int kTableGrid = 1024, kRowsGridMax = 4096;
 struct RowsCtl {
     int odd;                       // set by the rows, cleared by the table
-    int left;                      // whether the rows left the call (k_entry_table)
     int top[kTableGrid];           // the largest node id of each table workgroup's elements
     unsigned found[kRowsGridMax];  // table entries of each rows workgroup that are elements
+    int left;                      // whether the rows left the call (k_entry_lists)
 };
 
 // Whether the rows left a call of nE elements to what follows them: they found something odd,
@@ -150,25 +152,6 @@ __global__ void __launch_bounds__(kBlock)
     add_block<OP, PREC>(coord, coef, values, row, col, e2n, e2e, first + (int)(t >> 4), (int)(t & 15));
 }
 
-// Every color in one workgroup, for a call that the rows left to the colors.
-template <int OP, int PREC>
-__global__ void __launch_bounds__(1024)
-    k_assemble_colors_one(ColorOffsets co, const double *__restrict__ coord,
-                            const double *__restrict__ coef, double *values,
-                            const int *__restrict__ row, const int *__restrict__ col,
-                            const int4 *__restrict__ e2n, const int *__restrict__ e2e, int64_t nv,
-                            const RowsCtl *__restrict__ ctl, int groups)
-{
-    __shared__ unsigned long long s[1024];
-    if (!rows_verdict<1024>(ctl, groups, co.off[co.n], s)) return;
-    for (int64_t z = threadIdx.x; z < nv; z += 1024) values[z] = 0.0;
-    for (int c = 0; c < co.n; c++) {
-        __syncthreads();
-        for (int t = co.off[c] * 16 + threadIdx.x; t < co.off[c + 1] * 16; t += 1024)
-            add_block<OP, PREC>(coord, coef, values, row, col, e2n, e2e, t >> 4, t & 15);
-    }
-}
-
 // ---- the whole assembly row by row ------------------------------------------------------
 //
 // One launch per color reads and writes every CSR block once per element that holds it (an
@@ -189,10 +172,10 @@ __global__ void __launch_bounds__(1024)
 // whatever the ids. Without those lines the launch after the rows took such a call: ela 40^3
 // with ids eight times as far 62,000 us, so 337. All nodes by their rows' starts: lap 100^3
 // 1,560 -> 1,889, ela 60^3 353 -> 369.
-// What the rows cannot do is left to the launches after them, which otherwise return at once:
-// an elemToEdge entry outside its node's row or a diagonal entry that not all of the node's
-// elements share (k_entry_*), and, without elemToEdge, elements of one color that share a node,
-// elements that repeat one and rows of fewer entries (k_assemble_colors_one).
+// What the rows cannot do is left to the launches after them (k_entry_*, k_assemble_left), which
+// otherwise return at once: an elemToEdge entry outside its node's row, a diagonal entry that not
+// all of the node's elements share, elements that repeat a node, and, past the first nnz / 8
+// nodes, rows of fewer entries than an element's couplings.
 //
 // ela 60^3 1,830 -> 416 us, lap 31^3 with elemToEdge 148 -> 53 (the two prec
 // calls included); ela 60^3: k_row_table 63 us, k_assemble_rows 293.
@@ -227,11 +210,18 @@ __device__ __forceinline__ int line_of(int i, const int *__restrict__ row, int n
 
 __global__ void __launch_bounds__(kBlock)
     k_row_table(ColorOffsets co, const int4 *__restrict__ e2n, const int *__restrict__ row, int nE,
-                int nnz, int width, int *__restrict__ table, RowsCtl *__restrict__ ctl)
+                int nnz, int width, int *__restrict__ table, int *__restrict__ head,
+                RowsCtl *__restrict__ ctl)
 {
     __shared__ int smax[kBlock / 64];
     int top = 0;
     const int lane = threadIdx.x & 63;
+    // with elemToEdge, empty lists for k_entry_lists (here rather than in one more launch; head
+    // has a whole number of 16 bytes)
+    if (head)
+        for (int64_t z = (int64_t)blockIdx.x * kBlock + threadIdx.x; z < ((int64_t)nnz + 3) / 4;
+             z += (int64_t)gridDim.x * kBlock)
+            reinterpret_cast<int4 *>(head)[z] = make_int4(-1, -1, -1, -1);
     for (int64_t first = ((int64_t)blockIdx.x * kBlock + threadIdx.x) & ~63ll; first < nE;
          first += (int64_t)gridDim.x * kBlock) {
         const int e0 = __builtin_amdgcn_readfirstlane((int)first), e = e0 + lane;
@@ -604,51 +594,142 @@ __global__ void __launch_bounds__(64)
 
 // ---- any elemToEdge, entry by entry, for a call that the rows left
 //
-// The same table per CSR entry instead of per node: an entry receives at most one block of
-// each color. Nothing is assumed of the positions but that.
-__global__ void __launch_bounds__(kBlock)
-    k_entry_table(ColorOffsets co, const int *__restrict__ e2e, int nE, int nnz, int width,
-                  uint32_t *__restrict__ table, RowsCtl *__restrict__ ctl, int groups)
+// Every block is put into a list of its CSR entry, and a lane per entry sums its list in
+// ascending order of element and block: what the serial loop gives, whatever the positions are.
+// The lists lie in the bytes that held the rows' table. All positions reversed, ela 40^3: 757
+// us, with a slot per entry and color instead, in four times the workspace, 768.
+constexpr int kListGrid = 256, kListThreads = 512, kSumThreads = 128;
+
+__global__ void __launch_bounds__(kListThreads)
+    k_entry_lists(const int *__restrict__ e2e, int nE, int nnz, int *__restrict__ head,
+                  int *__restrict__ next, RowsCtl *__restrict__ ctl, int groups)
 {
-    __shared__ unsigned long long s[kBlock];
-    const bool left = rows_verdict<kBlock>(ctl, groups, nE, s);
+    __shared__ unsigned long long s[kListThreads];
+    const bool left = rows_verdict<kListThreads>(ctl, groups, nE, s);
     if (blockIdx.x == 0 && threadIdx.x == 0) ctl->left = left;
     if (!left) return;
-    const int lane = threadIdx.x & 63;
-    for (int64_t first = ((int64_t)blockIdx.x * kBlock + threadIdx.x) & ~63ll; first < (int64_t)nE * 16;
-         first += (int64_t)gridDim.x * kBlock) {
-        const int e0 = __builtin_amdgcn_readfirstlane((int)(first >> 4)), e = e0 + (lane >> 4);
-        const int c = color_of(co, e0, e, 4);
-        if (e >= nE) continue;
-        const int p = e2e[first + lane];
-        if (p >= 0 && p < nnz) table[(int64_t)p * width + c] = (uint32_t)e << 4 | (lane & 15);
+    const int64_t stride = (int64_t)gridDim.x * kListThreads;
+    for (int64_t t = (int64_t)blockIdx.x * kListThreads + threadIdx.x; t < (int64_t)nE * 4; t += stride) {
+        const int4 p = reinterpret_cast<const int4 *>(e2e)[t];
+        const int at[4] = {p.x, p.y, p.z, p.w};
+        int nx[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            nx[k] = at[k] >= 0 && at[k] < nnz ? atomicExch(head + at[k], (int)(t * 4 + k)) : -1;
+        reinterpret_cast<int4 *>(next)[t] = make_int4(nx[0], nx[1], nx[2], nx[3]);
     }
 }
 
 template <int OP, int PREC>
-__global__ void __launch_bounds__(kBlock)
-    k_entry_sum(ColorOffsets co, const double *__restrict__ coord, const double *__restrict__ coef,
-                double *__restrict__ values, const int4 *__restrict__ e2n,
-                const int *__restrict__ e2e, int nnz, int width,
-                const uint32_t *__restrict__ table, const RowsCtl *__restrict__ ctl)
+__global__ void __launch_bounds__(kSumThreads)
+    k_entry_sum(const double *__restrict__ coord, const double *__restrict__ coef,
+                double *__restrict__ values, const int4 *__restrict__ e2n, int nnz,
+                const int *__restrict__ head, const int *__restrict__ next,
+                const RowsCtl *__restrict__ ctl)
 {
     if (!ctl->left) return;
     constexpr int D = OP == MF_OP_ELA ? 9 : 1;
-    for (int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x; p < nnz; p += (int64_t)gridDim.x * kBlock) {
+    constexpr int SORT = 16;  // blocks sorted at a time
+    __shared__ int s_block[SORT][kSumThreads];
+    auto sorted = [&](int i) -> int & { return s_block[i][threadIdx.x]; };
+    for (int64_t p = (int64_t)blockIdx.x * kSumThreads + threadIdx.x; p < nnz;
+         p += (int64_t)gridDim.x * kSumThreads) {
         double acc[D];
 #pragma unroll
         for (int r = 0; r < D; r++) acc[r] = 0.0;
-        for (int c = 0; c < co.n; c++) {
-            const uint32_t t = table[p * width + c];
-            const int e = (int)(t >> 4), q = (int)(t & 15);
-            if (e < co.off[c] || e >= co.off[c + 1] || e2e[(int64_t)e * 16 + q] != p) continue;
-            double b[D];
-            elem_block<OP, PREC>(coord, coef, e2n[e], e, q, b);
+        for (int last = -1, n = SORT; n == SORT;) {
+            // the SORT lowest blocks past the last one
+            n = 0;
+            for (int t = head[p]; t >= 0; t = next[t]) {
+                if (t <= last || (n == SORT && t > sorted(SORT - 1))) continue;
+                int i = n < SORT ? n++ : SORT - 1;
+                for (; i > 0 && sorted(i - 1) > t; i--) sorted(i) = sorted(i - 1);
+                sorted(i) = t;
+            }
+            for (int i = 0; i < n; i++) {
+                last = sorted(i);
+                double b[D];
+                elem_block<OP, PREC>(coord, coef, e2n[last >> 4], last >> 4, last & 15, b);
 #pragma unroll
-            for (int r = 0; r < D; r++) acc[r] += b[r];
+                for (int r = 0; r < D; r++) acc[r] += b[r];
+            }
         }
 #pragma unroll
         for (int r = 0; r < D; r++) values[p * D + r] = acc[r];
+    }
+}
+
+// ---- the colors, for a call without elemToEdge that the rows left
+//
+// One launch that takes the colors in turn, and no workgroup waits for another: each owns every
+// kLeftGrid-th row, looks through all elements of a color for vertices of its own, and adds their
+// blocks once the color is listed, 16 lanes an element. Lanes of one element that share an entry
+// (a vertex stands twice in it) add in order, on one lane. Reading the elements kLeftGrid times is
+// what it costs: ela 40^3 with one element that repeats a vertex 1,045 us, one launch per color
+// 519, all colors in one workgroup 61,700.
+constexpr int kLeftGrid = 256, kLeftThreads = 1024;
+
+template <int OP, int PREC>
+__global__ void __launch_bounds__(kLeftThreads)
+    k_assemble_left(ColorOffsets co, const double *__restrict__ coord,
+                    const double *__restrict__ coef, double *values, const int *__restrict__ row,
+                    const int *__restrict__ col, const int4 *__restrict__ e2n, int nnz,
+                    const RowsCtl *__restrict__ ctl, int tables, int groups)
+{
+    constexpr int D = OP == MF_OP_ELA ? 9 : 1;
+    constexpr int PER = 4, STEP = PER * kLeftThreads, LIST = 2 * STEP;
+    __shared__ unsigned long long s[kLeftThreads];
+    if (!rows_verdict<kLeftThreads>(ctl, groups, co.off[co.n], s)) return;
+    __shared__ int s_list[LIST], s_n;
+    const int w = blockIdx.x, tid = threadIdx.x, l = tid & 15;
+    auto own = [&](int v) { return (unsigned)v % kLeftGrid == (unsigned)w; };
+    int N = 0;
+    for (int t = 0; t < tables; t++) N = N > ctl->top[t] ? N : ctl->top[t];
+    for (int64_t v = w + (int64_t)(tid >> 4) * kLeftGrid; v <= N; v += (kLeftThreads / 16) * kLeftGrid) {
+        if (v == 0) continue;
+        const int64_t a = (int64_t)(row[v - 1] > 0 ? row[v - 1] : 0) * D;
+        const int64_t b = (int64_t)(row[v] < nnz ? row[v] : nnz) * D;
+        for (int64_t z = a + l; z < b; z += 16) values[z] = 0.0;
+    }
+    if (tid == 0) s_n = 0;
+    for (int c = 0; c < co.n; c++) {
+        for (int64_t first = co.off[c]; first < co.off[c + 1]; first += STEP) {
+            __syncthreads();  // the list's places are free
+#pragma unroll
+            for (int u = 0; u < PER; u++) {
+                const int64_t e = first + u * kLeftThreads + tid;
+                if (e >= co.off[c + 1]) continue;
+                const int4 q = e2n[e];
+                if (own(q.x) || own(q.y) || own(q.z) || own(q.w)) s_list[atomicAdd(&s_n, 1)] = (int)e;
+            }
+            __syncthreads();
+            const int n = s_n;
+            if (n <= LIST - STEP && first + STEP < co.off[c + 1]) continue;
+            for (int i = tid >> 4; i < n; i += kLeftThreads / 16) {
+                const int e = s_list[i], j = l >> 2, k = l & 3;
+                const int4 q = e2n[e];
+                const int v[4] = {q.x, q.y, q.z, q.w};
+                const int nj = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
+                const int nk = k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
+                int p = own(nj) ? elem_position(row, col, nullptr, e, nj, nk, l) : -1;
+                if (p >= nnz) p = -1;
+                bool twice = false;
+#pragma unroll
+                for (int m = 1; m < 16; m++) twice |= p >= 0 && __shfl_xor(p, m, 16) == p;
+                const bool serial = (__ballot(twice) >> (tid & 48)) & 0xFFFFu;
+                for (int t = serial ? 0 : l; t < (serial ? 16 : l + 1); t++) {
+                    const int pt = serial ? __shfl(p, t, 16) : p;
+                    if (pt < 0 || (serial && l > 0)) continue;
+                    double b[D];
+                    elem_block<OP, PREC>(coord, coef, q, e, t, b);
+                    double *o = values + (int64_t)pt * D;
+#pragma unroll
+                    for (int r = 0; r < D; r++) o[r] += b[r];
+                }
+            }
+            __syncthreads();  // this color's sums, and the list, before the next one's
+            if (tid == 0) s_n = 0;
+        }
     }
 }
 
@@ -802,8 +883,6 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
         (void)hipGetLastError();
         return false;
     }
-    hipMemPool_t pool = mf::workspace_pool();
-    if (!pool) return false;
     ColorOffsets co;
     co.n = nbColors;
     std::memcpy(co.off, colorToElem, (size_t)(nbColors + 1) * sizeof(int));
@@ -814,38 +893,32 @@ bool launch_rows(const double *coord, const double *coef, double *values, const 
     constexpr int kPerCu = OP == MF_OP_ELA && PREC == MF_PREC_FP64 ? 8 : 16;
     static_assert(256 * kPerCu <= kRowsGridMax, "one slot per workgroup");
     const int groups = (int)std::min<int64_t>(256 * kPerCu, ((int64_t)nnz / 16 + 8) / 8 * 8);
-    const size_t head = (sizeof(RowsCtl) + 255) / 256 * 256;
-    const size_t bytes = head + (size_t)std::max(e2e ? nnz : 0, table_lines(nnz)) * width * sizeof(int);
-    unsigned char *buf = nullptr;
-    if (hipMallocFromPoolAsync(reinterpret_cast<void **>(&buf), bytes, pool, s) != hipSuccess) {
-        (void)hipGetLastError();
-        return false;
-    }
-    RowsCtl *ctl = reinterpret_cast<RowsCtl *>(buf);
-    int *table = reinterpret_cast<int *>(buf + head);
+    // the control block and the table, whose bytes then hold the lists of k_entry_lists, their
+    // heads before it
+    const size_t heads = e2e ? (size_t)nnz : 0;
+    const size_t slots = std::max((size_t)table_lines(nnz) * width, e2e ? (size_t)nbElem * 16 : 0);
+    mf::Workspace ws(mf::Workspace::padded(sizeof(RowsCtl)) + mf::Workspace::padded(heads * sizeof(int)) +
+                         mf::Workspace::padded(slots * sizeof(int)), s);
+    if (!ws.ok()) return false;
+    RowsCtl *ctl = ws.cut<RowsCtl>(1);
+    int *head = e2e ? ws.cut<int>(heads) : nullptr, *table = ws.cut<int>(slots);
     const int4 *en = reinterpret_cast<const int4 *>(e2n);
     hipLaunchKernelGGL(k_row_table, dim3((unsigned)tables), dim3(kBlock), 0, s, co, en, row, nbElem,
-                       nnz, width, table, ctl);
+                       nnz, width, table, head, ctl);
     if (e2e) {
         launch_rows_width<OP, PREC, true>(kc, co, coord, coef, values, row, col, en, e2e, nnz, table,
                                           ctl, tables, groups, s);
-        // any table of positions may be: these return at once unless the rows left the call
-        uint32_t *entries = reinterpret_cast<uint32_t *>(table);
-        hipLaunchKernelGGL(k_entry_table, dim3(256), dim3(kBlock), 0, s, co, e2e, nbElem, nnz, width,
-                           entries, ctl, groups);
-        hipLaunchKernelGGL((k_entry_sum<OP, PREC>), dim3(1024), dim3(kBlock), 0, s, co, coord, coef,
-                           values, en, e2e, nnz, width, entries, ctl);
+        hipLaunchKernelGGL(k_entry_lists, dim3(kListGrid), dim3(kListThreads), 0, s, e2e, nbElem, nnz,
+                           head, table, ctl, groups);
+        hipLaunchKernelGGL((k_entry_sum<OP, PREC>), dim3(2048), dim3(kSumThreads), 0, s, coord, coef,
+                           values, en, nnz, head, table, ctl);
     } else {
         launch_rows_width<OP, PREC, false>(kc, co, coord, coef, values, row, col, en, e2e, nnz, table,
                                            ctl, tables, groups, s);
-        // left: rows shorter than an element's couplings, a vertex that stands twice in an
-        // element, or an invalid coloring
-        hipLaunchKernelGGL((k_assemble_colors_one<OP, PREC>), dim3(1), dim3(1024), 0, s, co, coord,
-                           coef, values, row, col, en, e2e,
-                           (int64_t)nnz * (OP == MF_OP_ELA ? 9 : 1), ctl, groups);
+        hipLaunchKernelGGL((k_assemble_left<OP, PREC>), dim3(kLeftGrid), dim3(kLeftThreads), 0, s, co,
+                           coord, coef, values, row, col, en, nnz, ctl, tables, groups);
     }
-    const bool ok = hipGetLastError() == hipSuccess;
-    *status = hipFreeAsync(buf, s) == hipSuccess && ok ? MF_OK : MF_ERR_HIP;
+    *status = hipGetLastError() == hipSuccess ? MF_OK : MF_ERR_HIP;
     return true;
 }
 

@@ -189,3 +189,43 @@ def test_rows_of_a_part_that_keeps_global_ids(mf, gpu, op, far):
     rows, colors = times(mf, gpu, wide, row=row, col=col, e2n=e2n)
     print(f"  rows {rows:.3f} ms, colors {colors:.3f} ms", flush=True)
     assert rows < 2 * colors
+
+
+def serial(mf, gpu, orc, m, e2n, e2e=None, precision=0):
+    """(mf_assembly, the oracle's serial loop) with these elements and positions."""
+    D = gpu.DeviceArray.from_numpy
+    values = D(np.full(m.nnz * m.dim, np.nan))
+    gpu.assembly(D(m.coord), values, D(m.row), D(m.col), D(e2n), None if e2e is None else D(e2e),
+                 m.nbElem, m.nnz, m.dim, m.operatorID, m.colorToElem, coef=D(m.coef),
+                 precision=precision)
+    return values.numpy(), orc.assembly(m.coord, m.row, m.col, e2n, m.operatorID, coef=m.coef,
+                                        e2e=e2e, mixed=precision != 0)
+
+
+@pytest.mark.parametrize("op,precision,n", [(0, 0, 4), (1, 0, 9), (0, 1, 9), (1, 1, 4)])
+def test_left_calls_equal_the_serial_loop(mf, orc, gpu, op, precision, n):
+    """What the rows leave is summed in the order of the serial loop: elements that repeat a
+    vertex, and an elemToEdge of reversed entries."""
+    print(f"[left] op={op} precision={precision} n={n}", flush=True)
+    coord, e2n, code, nnz = mf.generate_cube(n, 0.25, 3, 11)
+    m = mf.Mesh(coord, e2n, code, nnz, op, coef=mf.generate_coef(op, e2n.size // 4, 9))
+    e2e = mf.create_elemToEdge(m.row, m.col, m.elemToNode)
+    repeats = m.elemToNode.copy()
+    repeats[3::4 * 7] = repeats[2::4 * 7]
+    for what, nodes, at in (("repeated vertices", repeats, None),
+                            ("repeated vertices, elemToEdge", repeats,
+                             mf.create_elemToEdge(m.row, m.col, repeats)),
+                            ("reversed entries", m.elemToNode, m.nnz - 1 - e2e)):
+        got, want = serial(mf, gpu, orc, m, nodes, at, precision)
+        assert np.array_equal(got, want, equal_nan=True), what
+
+
+def test_left_call_uses_the_whole_gpu(mf, gpu):
+    """One element that repeats a vertex does not make the call tens of times slower."""
+    coord, e2n, code, nnz = mf.generate_cube(30, 0.25, 3, 11)
+    m = mf.Mesh(coord, e2n, code, nnz, 1, coef=mf.generate_coef(1, e2n.size // 4, 9))
+    e2n = m.elemToNode.copy()
+    e2n[3] = e2n[2]
+    left, colors = times(mf, gpu, m, row=m.row, col=m.col, e2n=e2n)
+    print(f"[left] {left:.3f} ms, colors {colors:.3f} ms", flush=True)
+    assert left < 4 * colors
