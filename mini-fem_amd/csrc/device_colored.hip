@@ -7,7 +7,8 @@
 // order, i.e. the reference COLORING build's element order. What the rows cannot do goes on, in
 // the same order, in launches after them that ordinarily return at once (k_entry_* with
 // elemToEdge, else k_assemble_left). Under stream capture, without
-// memory for its workspace and for patterns thinner than the elements' couplings it is one
+// memory for its workspace, for patterns thinner than the elements' couplings and for large lap
+// meshes with elemToEdge it is one
 // launch per color with 16 lanes per element (one per element block): elements of one color
 // share no node, so their scatter-adds never touch the same CSR entry and each pass is
 // race-free and deterministic, in the same order.
@@ -871,13 +872,19 @@ void launch_rows_width(int kc, const ColorOffsets &co, const double *coord, cons
 // stream under capture, whose graph would have to own the workspace; no memory for the
 // table; element ids that do not leave the bits it needs; or fewer than two entries per
 // element, which a pattern of the elements' couplings has (2.4 to 2.5 on cubes and Delaunay
-// meshes) and one of, say, the diagonals alone has not.
+// meshes) and one of, say, the diagonals alone has not. Nor does lap with elemToEdge past
+// kLapEdgesElems elements take it: the colors add 8 bytes an entry without a search, and the rows
+// read elemToEdge in 16-byte pieces out of order (us, rows and colors: 60^3 396 and 433, 75^3 830
+// and 830, 80^3 1,037 and 1,006, 100^3 2,130 and 1,901; ela 90^3 1,639 and 5,574).
+constexpr int kLapEdgesElems = 2500000;
+
 template <int OP, int PREC>
 bool launch_rows(const double *coord, const double *coef, double *values, const int *row,
                  const int *col, const int *e2n, const int *e2e, int nbElem, int nnz,
                  const int *colorToElem, int nbColors, hipStream_t s, int *status)
 {
     if (nbElem >= 1 << 27 || nnz / 2 < nbElem) return false;
+    if (OP == MF_OP_LAP && e2e && nbElem > kLapEdgesElems) return false;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();

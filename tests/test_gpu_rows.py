@@ -229,3 +229,20 @@ def test_left_call_uses_the_whole_gpu(mf, gpu):
     left, colors = times(mf, gpu, m, row=m.row, col=m.col, e2n=e2n)
     print(f"[left] {left:.3f} ms, colors {colors:.3f} ms", flush=True)
     assert left < 4 * colors
+
+
+def test_large_lap_with_edges(mf, gpu):
+    """The first sizes that leave the rows for the launches per color (2.5 million elements)."""
+    print("[rows large]", flush=True)
+    coord, e2n, code, nnz = mf.generate_cube(76, 0.25, 3, 11)
+    m = mf.Mesh(coord, e2n, code, nnz, 0, coef=mf.generate_coef(0, e2n.size // 4, 9))
+    D = gpu.DeviceArray.from_numpy
+    dm = [D(x) for x in (m.coord, m.row, m.col, m.elemToNode, m.coef)]
+    e2e, values = D(mf.create_elemToEdge(m.row, m.col, m.elemToNode)), D(np.full(m.nnz, np.nan))
+    got = []
+    for edges in (None, e2e):
+        values.fill(np.nan)
+        gpu.assembly(dm[0], values, dm[1], dm[2], dm[3], edges, m.nbElem, m.nnz, 1, 0, m.colorToElem,
+                     coef=dm[4])
+        got.append(values.numpy())
+    same(got, "76^3")
