@@ -25,6 +25,9 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Two doubles as one 16-byte access at any multiple of 8 bytes, as a CSR row's values lie.
+using Two = double __attribute__((ext_vector_type(2), aligned(8)));
+
 // The current device's own pool of stream-ordered memory, for the workspaces of calls
 // (device_runtime.hip); null when it cannot be made. hipFreeAsync makes it safe for several
 // streams and threads.

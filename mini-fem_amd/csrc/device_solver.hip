@@ -204,7 +204,7 @@ __global__ void __launch_bounds__(kBT)
             const double *src = values + (int64_t)c0 * 9;
             for (int d = 2 * lane; d < nd; d += 128) {
                 if (d + 1 < nd) {
-                    const double2 v = *reinterpret_cast<const double2 *>(src + d);
+                    const mf::Two v = *reinterpret_cast<const mf::Two *>(src + d);
                     st[d] = v.x;
                     st[d + 1] = v.y;
                 } else {
@@ -426,10 +426,12 @@ __global__ void k_check_cols(const int *__restrict__ col, int64_t nnz, int N, in
 
 // New row t = old row order[t], its entries in their own order, columns renumbered, the
 // columns of fixed dofs zero (m: the mask in the new order): the product then gathers the
-// direction itself, and needs no masked copy of it. A row's values are one contiguous run on
-// both sides, moved by its 16 lanes in 16-byte pieces, five of a lane in flight (333 us for
-// ela 80^3, a block per lane word by word 386: rows of 1 KB in random order); the few columns
-// of fixed dofs are zeroed after them, by the same wave.
+// direction itself, and needs no masked copy of it. 16 lanes take a row 16 entries at a time:
+// each lane the column of one, then all of them the entries' values, one contiguous run on both
+// sides, in 16-byte pieces (the first read before the columns, so that both are in flight). A
+// piece asks the lanes of its entries for their masks and is stored once, as it is to stay
+// (311 us for ela 80^3; the pieces as they were read, fixed dofs zeroed by more stores, 325; a
+// block per lane word by word 386: rows of 1 KB in random order).
 template <int DD>
 __global__ void __launch_bounds__(kBT)
     k_order_csr(const int *__restrict__ order, const int *__restrict__ inv,
@@ -438,39 +440,47 @@ __global__ void __launch_bounds__(kBT)
                 const uint8_t *__restrict__ m, int N, int *__restrict__ colp,
                 double *__restrict__ valp)
 {
-    constexpr int CP = 5;
-    const int l = threadIdx.x % kGroup;
+    const int l = threadIdx.x % kGroup, g = (threadIdx.x >> 4) & 3;
     const int groups = gridDim.x * (kBT / kGroup);
     for (int t = blockIdx.x * (kBT / kGroup) + threadIdx.x / kGroup; t < N; t += groups) {
-        const int i = order[t], src = row[i], n = row[i + 1] - src, dst = rowp[t], nd = n * DD;
-        const double *from = values + (int64_t)src * DD;
-        double *to = valp + (int64_t)dst * DD;
-        for (int j0 = 2 * l; j0 < nd; j0 += 2 * kGroup * CP) {
-            double2 v[CP];
-#pragma unroll
-            for (int k = 0; k < CP; k++) {
-                const int j = j0 + 2 * kGroup * k;
-                if (j + 1 < nd) v[k] = *reinterpret_cast<const double2 *>(from + j);
-                else if (j < nd) v[k].x = from[j];
-            }
-#pragma unroll
-            for (int k = 0; k < CP; k++) {
-                const int j = j0 + 2 * kGroup * k;
-                if (j + 1 < nd) *reinterpret_cast<double2 *>(to + j) = v[k];
-                else if (j < nd) to[j] = v[k].x;
-            }
-        }
-        for (int k = l; k < n; k += kGroup) {
-            const int j = inv[col[src + k] - 1];
-            colp[dst + k] = j + 1;
-            const unsigned mj = m[j];
-            if (!mj) continue;
-            double *o = to + (int64_t)k * DD;
-            if constexpr (DD == 9) {
-                for (int e = 0; e < 3; e++)
-                    if ((mj >> e) & 1u) o[e] = o[3 + e] = o[6 + e] = 0.0;
+        const int i = order[t], src = row[i], n = row[i + 1] - src, dst = rowp[t];
+        for (int c0 = 0; c0 < n; c0 += kGroup) {
+            const bool on = c0 + l < n;
+            const double *from = values + (int64_t)(src + c0) * DD;
+            double *to = valp + (int64_t)(dst + c0) * DD;
+            if constexpr (DD == 1) {
+                const double v = on ? from[l] : 0.0;
+                const int j = on ? inv[col[src + c0 + l] - 1] : 0;
+                if (on) {
+                    colp[dst + c0 + l] = j + 1;
+                    to[l] = m[j] ? 0.0 : v;
+                }
             } else {
-                o[0] = 0.0;
+                constexpr int CP = (kGroup * DD / 2 + kGroup - 1) / kGroup;
+                const int nd = min(n - c0, kGroup) * DD;
+                mf::Two v[CP];
+#pragma unroll
+                for (int k = 0; k < CP; k++) {
+                    const int d = 2 * (l + kGroup * k);
+                    if (d + 1 < nd) v[k] = *reinterpret_cast<const mf::Two *>(from + d);
+                    else v[k] = mf::Two{d < nd ? from[d] : 0.0, 0.0};
+                }
+                const int j = on ? inv[col[src + c0 + l] - 1] : 0;
+                const unsigned mj = on ? m[j] : 0;
+                if (on) colp[dst + c0 + l] = j + 1;
+                const bool any = (__ballot(mj != 0) >> (16 * g)) & 0xFFFFu;
+#pragma unroll
+                for (int k = 0; k < CP; k++) {
+                    const int d = 2 * (l + kGroup * k);
+                    if (any) {  // entry d / 9, its column d % 3
+                        const unsigned a = __shfl(mj, min(d / 9, kGroup - 1), kGroup),
+                                       b = __shfl(mj, min((d + 1) / 9, kGroup - 1), kGroup);
+                        if ((a >> (d % 3)) & 1u) v[k].x = 0.0;
+                        if ((b >> ((d + 1) % 3)) & 1u) v[k].y = 0.0;
+                    }
+                    if (d + 1 < nd) *reinterpret_cast<mf::Two *>(to + d) = v[k];
+                    else if (d < nd) to[d] = v[k].x;
+                }
             }
         }
     }

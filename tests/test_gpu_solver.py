@@ -116,3 +116,35 @@ def test_pcg_ordered_rejects_a_bad_order(mf, gpu):
                     order=gpu.DeviceArray.from_numpy(bad.astype(np.int32)))
         assert exc.value.status == -1
         assert np.all(dx.numpy() == 7.0)
+
+
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("mesh", ["delaunay", "fan"])
+def test_pcg_ordered_copy_of_ragged_rows(mf, gpu, op, mesh):
+    """The copy takes a row 16 entries at a time and zeroes the columns of fixed dofs on the
+    way: rows of 7 to 30 entries, even and odd, and of 72, with every combination of a node's
+    dofs fixed. Two iterations from a start that is not zero at the fixed dofs, in a random
+    order and in the mesh's: the same x but for the order of the sums' terms (some thousand
+    roundings of 1e-16 in each of a few scalars)."""
+    import bench
+    from test_gpu_rows import fan
+    print(f"[pcg ragged] op={op} {mesh}", flush=True)
+    if mesh == "fan":
+        mesh = fan(70, op, mf)
+    else:
+        coord, e2n, code, nnz = bench.delaunay_arrays(700, seed=5)
+        mesh = mf.Mesh(coord, e2n, code, nnz, op, coef=mf.generate_coef(op, e2n.size // 4, 5))
+    n, d = mesh.nbNodes, 3 if op else 1
+    rng = np.random.default_rng(8)
+    mesh.checkBounds = (rng.random(3 * n) < 0.3).astype(np.int32)
+    plan, dm = gpu.Plan(mesh), gpu.DeviceMesh(mesh)
+    plan.assemble(dm.coord, dm.coef, dm.values, dm.prec)
+    b, x0 = rng.standard_normal(n * d), rng.standard_normal(n * d)
+    db, got = gpu.DeviceArray.from_numpy(b), []
+    for order in (None, gpu.DeviceArray.from_numpy(rng.permutation(n).astype(np.int32))):
+        dx = gpu.DeviceArray.from_numpy(x0)
+        it, _ = gpu.pcg(op, n, dm.row, dm.col, dm.values, dm.prec, dm.checkBounds, db, dx,
+                        rtol=1e-15, max_iter=2, order=order)
+        assert it == 2
+        got.append(dx.numpy())
+    assert np.linalg.norm(got[0] - got[1]) <= 1e-11 * np.linalg.norm(got[0])
