@@ -549,7 +549,7 @@ __global__ void __launch_bounds__(64)
                     if constexpr (ELA) {
 #pragma unroll
                         for (int q = 0; q < 4; q++)
-                            *reinterpret_cast<double2 *>(o + 2 * q) = make_double2(acc[2 * q], acc[2 * q + 1]);
+                            *reinterpret_cast<mf::Two *>(o + 2 * q) = mf::Two{acc[2 * q], acc[2 * q + 1]};
                         o[8] = acc[8];
                     } else {
                         o[0] = acc[0];
@@ -575,6 +575,7 @@ __global__ void __launch_bounds__(64)
             for (int o = 8; o > 0; o >>= 1) seen += __shfl_xor(seen, o, 16);
             mf::wave_sync();
             if (!__ballot(matched != seen)) break;
+            __threadfence();  // the second pass stores some of the first's entries from other lanes
         }
         r0 = r0n;
         r1 = r1n;
