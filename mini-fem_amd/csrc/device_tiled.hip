@@ -1221,6 +1221,7 @@ int launch_variant(mf_plan *p, const double *coord, const double *coef, double *
 struct Resolved {
     int budget, block, max_rows, slot64, slot32, id_chunks;
     bool float_stage;  // size the tiles by the float stage slot (mixed modes only)
+    bool alone;        // the second schedule may be made
 };
 
 int resolve_params(int op, const mf_plan_params *params, Resolved *r)
@@ -1232,7 +1233,9 @@ int resolve_params(int op, const mf_plan_params *params, Resolved *r)
     r->max_rows = 254;
     r->id_chunks = 1;
     r->float_stage = false;
+    r->alone = true;
     if (params) {
+        const Resolved own = *r;
         if (params->tile_lds_bytes > 0) r->budget = params->tile_lds_bytes;
         if (params->block_threads > 0) r->block = params->block_threads;
         if (params->max_tile_rows > 0) r->max_rows = params->max_tile_rows;
@@ -1241,6 +1244,9 @@ int resolve_params(int op, const mf_plan_params *params, Resolved *r)
         if (sp != MF_PREC_FP64 && sp != MF_PREC_MIXED && sp != MF_PREC_MIXED_F32COEF)
             return MF_ERR_ARG;
         r->float_stage = sp != MF_PREC_FP64;
+        // the second schedule goes with the library's own tile sizes only
+        r->alone = r->budget == own.budget && r->block == own.block &&
+                   r->max_rows == own.max_rows && r->id_chunks == own.id_chunks;
     }
     r->slot64 = mf::stage_len(ela, true) * 8;
     r->slot32 = mf::stage_len(ela, false) * 4;
@@ -1322,7 +1328,10 @@ bool valid_args(int op, int nE, int N, int nnz, const int *e2n, const int *row, 
            (nE == 0 || e2n) && row && (nnz == 0 || col);
 }
 
-using PlanGuard = std::unique_ptr<mf_plan, void (*)(mf_plan *)>;
+struct FreePlan {
+    void operator()(mf_plan *p) const { free_plan(p); }
+};
+using PlanGuard = std::unique_ptr<mf_plan, FreePlan>;
 
 // Builds a schedule (parts as in build_plan) on the host.
 int make_schedule(PlanGuard &guard, mf::PlanHost &h, int parts, const Resolved &r, int op, int nE,
@@ -1388,28 +1397,50 @@ int upload_schedule(mf_plan *p, const mf::PlanHost &h, const std::vector<int32_t
 // A launch of several plans keeps the default tiles: together they fill the CUs.
 constexpr int kAloneRounds = 2, kAloneRows = 12;
 
-int alone_parts(const mf::PlanHost &h, int *parts)
+int alone_parts(const mf::PlanHost &h, int cus)
 {
-    int dev = 0, cus = 0;
-    *parts = 0;
     const int T = (int)h.tiles.size(), rows = (int)h.tile_rowinfo.size();
-    if (T == 0) return MF_OK;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return MF_ERR_HIP;
+    if (T == 0) return 0;
     cus = std::max(1, cus / kXcd) * kXcd;
     const int rounds = (T + cus - 1) / cus;
-    if (rounds > kAloneRounds) return MF_OK;
+    if (rounds > kAloneRounds) return 0;
     int64_t sum = 0, most = 0;
     for (const mf::RowInfo &ri : h.tile_rowinfo) {
         const int val = (ri.inc >> 16) & 0xFFFF;
         sum += val;
         most = std::max<int64_t>(most, val);
     }
-    if (rounds > 1 && 2 * most * rows > 3 * sum) return MF_OK;
+    if (rounds > 1 && 2 * most * rows > 3 * sum) return 0;
     const int p = std::min(rounds * cus, rows / kAloneRows);
-    if (10 * (int64_t)T < 9 * (int64_t)p) *parts = p;
-    return MF_OK;
+    return 10 * (int64_t)T < 9 * (int64_t)p ? p : 0;
+}
+
+int device_cus()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+        return cus;
+    (void)hipGetLastError();
+    return 0;
+}
+
+// The second schedule of a plan whose first is h, on the host: null where none is of use, and
+// where anything fails, which leaves the plan as it is without it.
+PlanGuard make_alone(mf::PlanHost &ha, const mf::PlanHost &h, int cus, const Resolved &r, int op,
+                     int nE, int N, int nnz, const int *e2n, const int *row, const int *col,
+                     const int *checkBounds, const double *coord)
+{
+    PlanGuard alone;
+    const int parts = r.alone && coord && cus > 0 ? alone_parts(h, cus) : 0;
+    if (parts == 0) return alone;
+    int st = MF_ERR_STATE;
+    try {
+        st = make_schedule(alone, ha, parts, r, op, nE, N, nnz, e2n, row, col, checkBounds, coord);
+    } catch (...) {
+    }
+    if (st != MF_OK || (int)ha.tiles.size() > parts) alone.reset();
+    return alone;
 }
 
 }  // namespace
@@ -1427,21 +1458,12 @@ extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nb
         int st = resolve_params(operatorID, params, &r);
         if (st != MF_OK) return st;
         mf::PlanHost h, ha;
-        PlanGuard guard(nullptr, free_plan), alone(nullptr, free_plan);
+        PlanGuard guard;
         st = make_schedule(guard, h, 0, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
                            checkBounds, coord);
         if (st != MF_OK) return st;
-        // the second schedule, with the library's own tile sizes only
-        Resolved own;
-        (void)resolve_params(operatorID, nullptr, &own);
-        const bool sized = r.budget != own.budget || r.block != own.block ||
-                           r.max_rows != own.max_rows || r.id_chunks != own.id_chunks;
-        int parts = 0;
-        if (!sized && coord) st = alone_parts(h, &parts);
-        if (st == MF_OK && parts > 0)
-            st = make_schedule(alone, ha, parts, r, operatorID, nbElem, nbNodes, nnz, elemToNode,
-                               row, col, checkBounds, coord);
-        if (st != MF_OK) return st;
+        PlanGuard alone = make_alone(ha, h, r.alone ? device_cus() : 0, r, operatorID, nbElem,
+                                     nbNodes, nnz, elemToNode, row, col, checkBounds, coord);
 
         // Every host container is built before the first device allocation, and the plan is
         // held by a guard until it is complete: an exception thrown here (bad_alloc) releases
@@ -1453,15 +1475,11 @@ extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nb
             cbHost.assign(checkBounds, checkBounds + (size_t)nbNodes * 3);
         st = upload_schedule(guard.get(), h, cbHost);
         if (st != MF_OK) return st;
-        if (alone && (int)ha.tiles.size() <= parts) {
-            // without room for it the plan does without
-            st = upload_schedule(alone.get(), ha, cbHost);
-            if (st == MF_OK)
+        if (alone) {
+            if (upload_schedule(alone.get(), ha, cbHost) == MF_OK)
                 guard->alone = alone.release();
-            else if (st == MF_ERR_NOMEM)
+            else  // no room for it: the plan does without
                 (void)hipGetLastError();
-            else
-                return st;
         }
         *plan = guard.release();
         return MF_OK;
