@@ -340,8 +340,20 @@ int mf_plan_host_stats(int operatorID, int nbElem, int nbNodes, int nnz,
 /* Plan statistics: out[0] tiles, [1] tile-element slots, [2] off-diagonal tasks
  * (a pair computed once counts once), [3] incidence entries, [4] plan bytes on the
  * device, [5] LDS bytes per workgroup (in the stage precision), [6] threads per
- * workgroup, [7] rows per tile (max). */
+ * workgroup, [7] rows per tile (max). Of the default tiles; a second schedule's bytes come
+ * on top. */
 int mf_plan_stats(const mf_plan *plan, int64_t out[8]);
+
+/* The same of the schedule that mf_plan_assemble runs: the second one's where the plan holds
+ * one, else those of mf_plan_stats. */
+int mf_plan_alone_stats(const mf_plan *plan, int64_t out[8]);
+
+/* What mf_plan_alone_stats would report on a GPU of computeUnits, the schedules built and
+ * validated on the host only. */
+int mf_plan_host_alone_stats(int operatorID, int nbElem, int nbNodes, int nnz,
+                             const int *elemToNode, const int *row, const int *col,
+                             const double *coord, const mf_plan_params *params, int computeUnits,
+                             int64_t out[8]);
 
 /* The plan's node order (device, N ints, 0-based): the rows of its tiles in tile order
  * (the rows of a tile are spatially close), then the nodes with an empty row; a

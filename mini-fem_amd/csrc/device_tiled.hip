@@ -1513,6 +1513,34 @@ extern "C" int mf_plan_destroy(mf_plan *plan)
     return MF_OK;
 }
 
+extern "C" int mf_plan_host_alone_stats(int operatorID, int nbElem, int nbNodes, int nnz,
+                                        const int *elemToNode, const int *row, const int *col,
+                                        const double *coord, const mf_plan_params *params,
+                                        int computeUnits, int64_t out[8])
+{
+    return mf_guarded([&]() -> int {
+        if (!out || computeUnits < 1 ||
+            !valid_args(operatorID, nbElem, nbNodes, nnz, elemToNode, row, col))
+            return MF_ERR_ARG;
+        Resolved r;
+        int st = resolve_params(operatorID, params, &r);
+        if (st != MF_OK) return st;
+        mf::PlanHost h, ha;
+        PlanGuard plan;
+        st = make_schedule(plan, h, 0, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
+                           nullptr, coord);
+        if (st != MF_OK) return st;
+        const PlanGuard alone = make_alone(ha, h, computeUnits, r, operatorID, nbElem, nbNodes, nnz,
+                                           elemToNode, row, col, nullptr, coord);
+        return mf_plan_stats(alone ? alone.get() : plan.get(), out);
+    });
+}
+
+extern "C" int mf_plan_alone_stats(const mf_plan *plan, int64_t out[8])
+{
+    return mf_plan_stats(plan && plan->alone ? plan->alone : plan, out);
+}
+
 extern "C" int mf_plan_stats(const mf_plan *plan, int64_t out[8])
 {
     if (!plan || !out) return MF_ERR_ARG;

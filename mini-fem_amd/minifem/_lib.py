@@ -97,10 +97,12 @@ SIGNATURES = {
     "mf_plan_create": (_i, [_p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p]),
     "mf_plan_destroy": (_i, [_p]),
     "mf_plan_stats": (_i, [_p, _p]),
+    "mf_plan_alone_stats": (_i, [_p, _p]),
     "mf_plan_row_order": (_i, [_p, _p, _p]),
     "mf_plan_assemble": (_i, [_p, _p, _p, _p, _p, _i, _p, _p]),
     "mf_plan_write_probe": (_i, [_p, _p, _i, _p]),
     "mf_plan_host_stats": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _p]),
+    "mf_plan_host_alone_stats": (_i, [_i, _i, _i, _i, _p, _p, _p, _p, _p, _i, _p]),
     "mf_plans_assemble": (_i, [_p, _i, _i, _p]),
     "mf_plans_lds_bytes": (_i, [_p, _i, _i]),
     "mf_server_create": (_i, [_p, _p, _i64, _i, _i, _i]),

@@ -420,9 +420,11 @@ class Plan:
             ctypes.byref(params)), "mf_plan_create")
         self.ptr = p.value
 
-    def stats(self):
+    def stats(self, alone=False):
+        """The default tiles' statistics; alone: of the schedule that assemble() runs."""
         out = np.zeros(8, np.int64)
-        check(self._lib.mf_plan_stats(self.ptr, out.ctypes.data), "mf_plan_stats")
+        fn = self._lib.mf_plan_alone_stats if alone else self._lib.mf_plan_stats
+        check(fn(self.ptr, out.ctypes.data), "mf_plan_stats")
         keys = ["tiles", "tile_elems", "tasks", "incidences", "plan_bytes", "lds_bytes",
                 "block_threads", "max_rows"]
         return dict(zip(keys, (int(x) for x in out)))

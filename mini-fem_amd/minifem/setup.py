@@ -246,8 +246,10 @@ class Mesh:
 
 
 def plan_host_stats(mesh, tile_lds_bytes=0, block_threads=0, max_tile_rows=0, use_coord=True,
-                    partition_coord=None, id_chunks=0, stage_precision=0):
-    """Builds and validates the tiled gather schedule on the host (mf_plan_host_stats).
+                    partition_coord=None, id_chunks=0, stage_precision=0, compute_units=0):
+    """Builds and validates the tiled gather schedule on the host (mf_plan_host_stats); with
+    compute_units, also the second schedule that a plan of its own launch would have on a GPU
+    of that many, whose statistics it then returns (mf_plan_host_alone_stats).
     partition_coord: coordinates used only to group nodes into tiles (default: the mesh's).
     stage_precision: the precision mode the tiles are sized for (0: FP64)."""
     import ctypes
@@ -259,10 +261,13 @@ def plan_host_stats(mesh, tile_lds_bytes=0, block_threads=0, max_tile_rows=0, us
     if pc.size != 3 * mesh.nbNodes:
         raise ValueError(f"partition_coord has {pc.size} values, the mesh needs "
                          f"{3 * mesh.nbNodes} (x, y, z per node)")
-    check(lib().mf_plan_host_stats(mesh.operatorID, mesh.nbElem, mesh.nbNodes, mesh.nnz,
-                                   _ptr(mesh.elemToNode), _ptr(mesh.row), _ptr(mesh.col),
-                                   _ptr(pc) if use_coord else None,
-                                   ctypes.byref(params), out.ctypes.data), "mf_plan_host_stats")
+    args = [mesh.operatorID, mesh.nbElem, mesh.nbNodes, mesh.nnz, _ptr(mesh.elemToNode),
+            _ptr(mesh.row), _ptr(mesh.col), _ptr(pc) if use_coord else None, ctypes.byref(params)]
+    if compute_units:
+        check(lib().mf_plan_host_alone_stats(*args, int(compute_units), out.ctypes.data),
+              "mf_plan_host_alone_stats")
+    else:
+        check(lib().mf_plan_host_stats(*args, out.ctypes.data), "mf_plan_host_stats")
     keys = ["tiles", "tile_elems", "tasks", "incidences", "plan_bytes", "lds_bytes",
             "block_threads", "max_rows"]
     return dict(zip(keys, (int(x) for x in out)))

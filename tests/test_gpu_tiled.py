@@ -438,3 +438,16 @@ def test_rows_at_every_place_in_a_line(mf, orc, gpu, precision, offset):
     ov = om.assemble(mixed=precision != 0)
     assert np.array_equal(got[start:start + n], ov)
     assert np.all(got[:start] == -1.0) and np.all(got[start + n:] == -1.0)
+
+
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("n,second", [(2, False), (9, True), (24, True), (28, True), (38, False)])
+def test_plans_that_hold_a_second_schedule(mf, gpu, op, n, second):
+    """The sizes whose plans run smaller tiles in a launch of their own: what the GPU's own
+    number of CUs gives is what the host says for 256."""
+    from minifem.setup import plan_host_stats
+    mesh = mf.Mesh.cube(n, 0.25, 3, op)
+    plan = gpu.Plan(mesh)
+    assert plan.stats() == plan_host_stats(mesh)
+    assert plan.stats(alone=True) == plan_host_stats(mesh, compute_units=256)
+    assert (plan.stats(alone=True)["tiles"] > plan.stats()["tiles"]) == second

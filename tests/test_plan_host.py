@@ -143,3 +143,21 @@ def test_plan_rejects_valence_above_128(mf):
     m.elemToNode, m.row, m.col, m.coord = e2n, row, col, coord
     with pytest.raises(mf.MiniFemError):
         plan_host_stats(m)
+
+
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("n,tiles", [(2, None), (3, 2), (9, 60), (20, 256), (24, 256), (30, 512), (38, None)])
+def test_second_schedule(mf, op, n, tiles):
+    """The smaller tiles of a launch of its own, built and validated on the host: a tile a CU
+    and round, but of no fewer than 12 rows; none where the default tiles already are as many
+    or go past two rounds; none beside sizes that the caller names, and without coordinates."""
+    coord, e2n, code, nnz = mf.generate_cube(n, 0.25, 3, 7)
+    m = mf.Mesh(coord, e2n, code, nnz, op)
+    default, alone = plan_host_stats(m), plan_host_stats(m, compute_units=256)
+    if tiles is None:
+        assert alone == default
+    else:
+        assert default["tiles"] < 0.9 * alone["tiles"] and alone["tiles"] == tiles
+        assert alone["lds_bytes"] < default["lds_bytes"]
+    for kw in ({"max_tile_rows": 200}, {"use_coord": False}):
+        assert plan_host_stats(m, compute_units=256, **kw) == plan_host_stats(m, **kw)
