@@ -1258,8 +1258,8 @@ int resolve_params(int op, const mf_plan_params *params, Resolved *r)
 
 int build_checked(mf::PlanHost &h, int op, int nE, int N, int nnz, const int *e2n,
                   const int *row, const int *col, const int *cb, const double *coord,
-                  const Resolved &r, int parts, int *lds64, int *lds32, int *back64 = nullptr,
-                  int *back32 = nullptr)
+                  const Resolved &r, int parts, const mf::PlanHost *same, int *lds64, int *lds32,
+                  int *back64 = nullptr, int *back32 = nullptr)
 {
     // the stage slot the tiles are sized by: a float-staged plan's FP64 layout may exceed
     // one CU's LDS, and that plan never launches in FP64
@@ -1286,7 +1286,7 @@ int build_checked(mf::PlanHost &h, int op, int nE, int N, int nnz, const int *e2
     int st = MF_OK, budget = r.budget;
     for (int cut = 0;; cut++) {
         st = mf::build_plan(h, op, nE, N, nnz, e2n, row, col, cb, coord, budget, r.max_rows, slot,
-                            r.block, r.id_chunks, parts);
+                            r.block, r.id_chunks, parts, same);
         if (st != MF_OK) return st;
         measure();
         const int over = (r.float_stage ? m32 : m64) + 16 - mf::kMaxLdsBytes;
@@ -1333,14 +1333,14 @@ struct FreePlan {
 };
 using PlanGuard = std::unique_ptr<mf_plan, FreePlan>;
 
-// Builds a schedule (parts as in build_plan) on the host.
-int make_schedule(PlanGuard &guard, mf::PlanHost &h, int parts, const Resolved &r, int op, int nE,
-                  int N, int nnz, const int *e2n, const int *row, const int *col,
-                  const int *checkBounds, const double *coord)
+// Builds a schedule (parts and same as in build_plan) on the host.
+int make_schedule(PlanGuard &guard, mf::PlanHost &h, int parts, const mf::PlanHost *same,
+                  const Resolved &r, int op, int nE, int N, int nnz, const int *e2n,
+                  const int *row, const int *col, const int *checkBounds, const double *coord)
 {
     int lds64 = 0, lds32 = 0, back64 = 0, back32 = 0;
     const int st = build_checked(h, op, nE, N, nnz, e2n, row, col, checkBounds, coord, r, parts,
-                                 &lds64, &lds32, &back64, &back32);
+                                 same, &lds64, &lds32, &back64, &back32);
     if (st != MF_OK) return st;
     guard.reset(new mf_plan);
     mf_plan *p = guard.get();
@@ -1436,7 +1436,7 @@ PlanGuard make_alone(mf::PlanHost &ha, const mf::PlanHost &h, int cus, const Res
     if (parts == 0) return alone;
     int st = MF_ERR_STATE;
     try {
-        st = make_schedule(alone, ha, parts, r, op, nE, N, nnz, e2n, row, col, checkBounds, coord);
+        st = make_schedule(alone, ha, parts, &h, r, op, nE, N, nnz, e2n, row, col, checkBounds, coord);
     } catch (...) {
     }
     if (st != MF_OK || (int)ha.tiles.size() > parts) alone.reset();
@@ -1459,7 +1459,7 @@ extern "C" int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nb
         if (st != MF_OK) return st;
         mf::PlanHost h, ha;
         PlanGuard guard;
-        st = make_schedule(guard, h, 0, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
+        st = make_schedule(guard, h, 0, nullptr, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
                            checkBounds, coord);
         if (st != MF_OK) return st;
         PlanGuard alone = make_alone(ha, h, r.alone ? device_cus() : 0, r, operatorID, nbElem,
@@ -1500,7 +1500,7 @@ extern "C" int mf_plan_host_stats(int operatorID, int nbElem, int nbNodes, int n
         mf::PlanHost h;
         int lds64 = 0, lds32 = 0;
         st = build_checked(h, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col, nullptr,
-                           coord, r, 0, &lds64, &lds32);
+                           coord, r, 0, nullptr, &lds64, &lds32);
         if (st != MF_OK) return st;
         fill_stats(h, r.float_stage ? lds32 : lds64, r.block, out);
         return MF_OK;
@@ -1527,7 +1527,7 @@ extern "C" int mf_plan_host_alone_stats(int operatorID, int nbElem, int nbNodes,
         if (st != MF_OK) return st;
         mf::PlanHost h, ha;
         PlanGuard plan;
-        st = make_schedule(plan, h, 0, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
+        st = make_schedule(plan, h, 0, nullptr, r, operatorID, nbElem, nbNodes, nnz, elemToNode, row, col,
                            nullptr, coord);
         if (st != MF_OK) return st;
         const PlanGuard alone = make_alone(ha, h, computeUnits, r, operatorID, nbElem, nbNodes, nnz,

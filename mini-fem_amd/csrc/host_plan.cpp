@@ -574,7 +574,8 @@ struct Emitter {
 
 int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, const int *row,
                const int *col, const int *checkBounds, const double *coord, int lds_budget,
-               int max_rows, int slot_bytes, int block, int id_chunks, int parts)
+               int max_rows, int slot_bytes, int block, int id_chunks, int parts,
+               const PlanHost *same)
 {
     p = PlanHost{};
     p.op = op;
@@ -595,9 +596,13 @@ int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, cons
         else rowsAll.push_back(i);
     }
     // each node's elements, ascending (the threaded counting fill of the setup)
-    std::vector<int> n2eI((size_t)N + 1, 0), n2eV((size_t)nE * 4 + 1);
-    const int st = mf_create_nodeToElem(e2n, nE, N, n2eI.data(), n2eV.data());
-    if (st != MF_OK) return st;
+    if (!same) {
+        p.n2eI.assign((size_t)N + 1, 0);
+        p.n2eV.resize((size_t)nE * 4 + 1);
+        const int st = mf_create_nodeToElem(e2n, nE, N, p.n2eI.data(), p.n2eV.data());
+        if (st != MF_OK) return st;
+    }
+    const std::vector<int> &n2eI = same ? same->n2eI : p.n2eI, &n2eV = same ? same->n2eV : p.n2eV;
     int maxVal = 0;
     for (int i = 0; i < N; i++) maxVal = std::max(maxVal, n2eI[i + 1] - n2eI[i]);
     if (maxVal > kMaxValence) return MF_ERR_ARG;

@@ -230,6 +230,7 @@ struct PlanHost {
     std::vector<uint32_t> task_rec;    // 4 words per task
     std::vector<int32_t> isolated;     // nodes with an empty row (no element)
     int max_node = 0, max_elem = 0, max_rows = 0;
+    std::vector<int> n2eI, n2eV;       // each node's elements, ascending (host only)
 };
 
 // Builds the schedule. coord (3N doubles) may be null: nodes are then ordered by a
@@ -240,10 +241,12 @@ struct PlanHost {
 // id_chunks > 1: the rows are first cut into that many contiguous node-id ranges, and
 // each range is bisected on its own (tiles then hold rows of one id range, so the tiles
 // that run at the same time write nearby CSR rows). parts > 1 (with coord): as many tiles of
-// nearly equal size, more only where one of them would not fit.
+// nearly equal size, more only where one of them would not fit. same: another plan of the same
+// mesh, whose node lists serve again.
 int build_plan(PlanHost &p, int op, int nE, int N, int nnz, const int *e2n, const int *row,
                const int *col, const int *checkBounds, const double *coord, int lds_budget,
-               int max_rows, int slot_bytes, int block, int id_chunks = 1, int parts = 0);
+               int max_rows, int slot_bytes, int block, int id_chunks = 1, int parts = 0,
+               const PlanHost *same = nullptr);
 
 // Checks every index the kernel will follow against the array it indexes, that every
 // CSR entry is written exactly once (diagonal, task or transpose) and that every task's
