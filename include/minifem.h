@@ -311,6 +311,8 @@ typedef struct mf_plan_params {
                              takes a little less LDS (ela 100^3: 1 % fewer tiles);
                              the plan then runs the two mixed modes only, and FP64 launches
                              of it (mf_plan_assemble, mf_plans_assemble) return MF_ERR_ARG */
+    int default_tiles;    /* nonzero: no second schedule (see mf_plan_create), for a plan that
+                             runs in mf_plans_assemble or a few times only */
 } mf_plan_params;
 
 /* Host arrays: elemToNode (color-permuted, 1-based, 4nE), row[N+1], col[nnz],
@@ -323,8 +325,11 @@ typedef struct mf_plan_params {
  * build runs on up to 16 host threads (environment MF_PLAN_THREADS sets the count); the
  * plan does not depend on the count. A small plan (tile_lds_bytes, block_threads,
  * max_tile_rows and id_chunks at their defaults; coord given; too few tiles for the GPU's CUs) holds
- * a second schedule of smaller tiles, which mf_plan_assemble runs: same results. The
- * calls that describe a plan and mf_plans_assemble use the default tiles. */
+ * a second schedule of smaller tiles, which mf_plan_assemble runs: same results. Making it
+ * takes about as long again as the plan (9^3 nodes 1.5 ms without and 2.6 with it, 30^3 14 and
+ * 23) and saves 1 to 4 us a launch; default_tiles leaves it out, as does a plan that has no
+ * memory for it. The other calls that describe a plan and mf_plans_assemble use the default
+ * tiles. */
 int mf_plan_create(mf_plan **plan, int operatorID, int nbElem, int nbNodes, int nnz,
                    const int *elemToNode, const int *row, const int *col,
                    const int *checkBounds, const double *coord,

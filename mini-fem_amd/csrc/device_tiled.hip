@@ -1245,7 +1245,7 @@ int resolve_params(int op, const mf_plan_params *params, Resolved *r)
             return MF_ERR_ARG;
         r->float_stage = sp != MF_PREC_FP64;
         // the second schedule goes with the library's own tile sizes only
-        r->alone = r->budget == own.budget && r->block == own.block &&
+        r->alone = !params->default_tiles && r->budget == own.budget && r->block == own.block &&
                    r->max_rows == own.max_rows && r->id_chunks == own.id_chunks;
     }
     r->slot64 = mf::stage_len(ela, true) * 8;

@@ -140,6 +140,7 @@ class Batch:
         do not fit one CU's LDS together, they are rebuilt with the tile budget lowered by
         the overflow."""
         params = dict(plan_params)
+        params.setdefault("default_tiles", True)  # they run in plans_assemble only
         for _ in range(3):
             plans = [gpu.Plan(u.mesh, partition_coord=u.partition_coord, **params)
                      for u in self.unions]

@@ -129,6 +129,8 @@ class Server:
         self.dms = [gpu.DeviceMesh(m) for m in self.meshes]
         self._plan_params = dict(plan_params or {})
         self._plan_params.setdefault("stage_precision", precision)
+        # every request runs in mf_plans_assemble, which takes the default tiles
+        self._plan_params.setdefault("default_tiles", True)
         self.plans = [gpu.Plan(m, **self._plan_params) for m in self.meshes]
         self.budget = int(hbm_budget)
         self.arena_mem = gpu.DeviceArray(self.budget, np.uint8)

@@ -246,7 +246,8 @@ class Mesh:
 
 
 def plan_host_stats(mesh, tile_lds_bytes=0, block_threads=0, max_tile_rows=0, use_coord=True,
-                    partition_coord=None, id_chunks=0, stage_precision=0, compute_units=0):
+                    partition_coord=None, id_chunks=0, stage_precision=0, compute_units=0,
+                    default_tiles=False):
     """Builds and validates the tiled gather schedule on the host (mf_plan_host_stats); with
     compute_units, also the second schedule that a plan of its own launch would have on a GPU
     of that many, whose statistics it then returns (mf_plan_host_alone_stats).
@@ -255,7 +256,7 @@ def plan_host_stats(mesh, tile_lds_bytes=0, block_threads=0, max_tile_rows=0, us
     import ctypes
     from ._lib import PlanParams
     params = PlanParams(int(tile_lds_bytes), int(block_threads), int(max_tile_rows),
-                        int(id_chunks), int(stage_precision))
+                        int(id_chunks), int(stage_precision), int(bool(default_tiles)))
     out = np.zeros(8, np.int64)
     pc = mesh.coord if partition_coord is None else _c(partition_coord, np.float64).ravel()
     if pc.size != 3 * mesh.nbNodes:

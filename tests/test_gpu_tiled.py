@@ -451,3 +451,24 @@ def test_plans_that_hold_a_second_schedule(mf, gpu, op, n, second):
     assert plan.stats() == plan_host_stats(mesh)
     assert plan.stats(alone=True) == plan_host_stats(mesh, compute_units=256)
     assert (plan.stats(alone=True)["tiles"] > plan.stats()["tiles"]) == second
+
+
+@pytest.mark.parametrize("op", [0, 1])
+def test_default_tiles_alone(mf, gpu, op):
+    """A plan made with default_tiles, and those of a server and of a union batch, which launch
+    several plans at once, hold no second schedule; same results."""
+    from minifem.batched import Batch
+    from minifem.serve import Server
+    mesh = mf.Mesh.cube(9, 0.25, 3, op, coef_seed=4)
+    dm, got = gpu.DeviceMesh(mesh), []
+    plans = [gpu.Plan(mesh), gpu.Plan(mesh, default_tiles=True)]
+    assert plans[0].stats(alone=True) != plans[0].stats() == plans[1].stats(alone=True)
+    for plan in plans:
+        dm.values.fill(np.nan)
+        plan.assemble(dm.coord, dm.coef, dm.values, dm.prec)
+        got.append(dm.values.numpy())
+    assert np.array_equal(got[0], got[1])
+    server = Server([mesh], 1 << 24)
+    server.add_mesh(mesh)
+    for plan in server.plans + Batch([mesh, mesh], union=True).plans:
+        assert plan.stats(alone=True) == plan.stats()
