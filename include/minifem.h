@@ -193,6 +193,14 @@ int mf_memcpy_d2h_async(void *dst, const void *src, size_t bytes, void *stream);
 int mf_event_query(void *event, int *done);
 int mf_stream_wait_event(void *stream, void *event);
 
+/* Calls that need workspace (mf_assembly, mf_pcg, the device setup) take it, in stream order,
+ * from a pool of the library's own, one per GPU, that keeps up to 2 GiB between them.
+ * mf_workspace_bytes: what the current GPU's pool holds. mf_workspace_release waits for that GPU and
+ * gives back all that no call is using; mf_dev_alloc and mf_plan_create do so themselves before
+ * they report that there is no memory. */
+int mf_workspace_bytes(int64_t *bytes);
+int mf_workspace_release(void);
+
 /* Stream capture into an executable HIP graph: mf_graph_begin(stream), enqueue work
  * (e.g. one mf_plan_assemble per mesh of a batch) on that stream, mf_graph_end(stream,
  * &graph); mf_graph_launch replays the whole batch as one submission. The captured

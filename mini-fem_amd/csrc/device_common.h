@@ -33,6 +33,10 @@ using Two = double __attribute__((ext_vector_type(2), aligned(8)));
 // streams and threads.
 hipMemPool_t workspace_pool();
 
+// hipMalloc that, where memory is short, has that pool give back what it keeps and tries once
+// more; a failure leaves no error behind.
+int device_alloc(void **ptr, size_t bytes);
+
 // One block of workspace, taken from the pool on construction and given back, in stream
 // order, on destruction. Pieces are cut from it in turn, 256-byte aligned.
 class Workspace {

@@ -74,7 +74,38 @@ hipMemPool_t workspace_pool()
     return pools[dev];
 }
 
+int device_alloc(void **ptr, size_t bytes)
+{
+    if (hipMalloc(ptr, bytes) == hipSuccess) return MF_OK;
+    (void)hipGetLastError();
+    if (mf_workspace_release() == MF_OK && hipMalloc(ptr, bytes) == hipSuccess) return MF_OK;
+    (void)hipGetLastError();
+    *ptr = nullptr;
+    return MF_ERR_NOMEM;
+}
+
 }  // namespace mf
+
+extern "C" int mf_workspace_bytes(int64_t *bytes)
+{
+    if (!bytes) return MF_ERR_ARG;
+    hipMemPool_t pool = mf::workspace_pool();
+    uint64_t held = 0;
+    if (!pool || hipMemPoolGetAttribute(pool, hipMemPoolAttrReservedMemCurrent, &held) != hipSuccess) {
+        (void)hipGetLastError();
+        return MF_ERR_HIP;
+    }
+    *bytes = (int64_t)held;
+    return MF_OK;
+}
+
+extern "C" int mf_workspace_release(void)
+{
+    hipMemPool_t pool = mf::workspace_pool();
+    if (pool && hipDeviceSynchronize() == hipSuccess && hipMemPoolTrimTo(pool, 0) == hipSuccess) return MF_OK;
+    (void)hipGetLastError();
+    return MF_ERR_HIP;
+}
 
 extern "C" int mf_gather_probe(double *dst, const double *src, const int64_t *idx, int64_t n,
                                void *stream)
@@ -106,7 +137,7 @@ extern "C" int mf_dev_alloc(void **ptr, size_t bytes)
     if (!ptr) return MF_ERR_ARG;
     *ptr = nullptr;
     if (bytes == 0) bytes = 1;
-    return hipMalloc(ptr, bytes) == hipSuccess ? MF_OK : MF_ERR_NOMEM;
+    return mf::device_alloc(ptr, bytes);
 }
 
 extern "C" int mf_dev_free(void *ptr)

@@ -559,7 +559,7 @@ struct StreamDrain {
 
 inline int dev_alloc(DevBuf &b, size_t bytes)
 {
-    return hipMalloc(&b.p, std::max<size_t>(bytes, 16)) == hipSuccess ? MF_OK : MF_ERR_NOMEM;
+    return mf::device_alloc(&b.p, std::max<size_t>(bytes, 16));
 }
 
 // The device arrays of one coloring.

@@ -1113,7 +1113,7 @@ int upload(T **dst, const std::vector<T> &src)
 {
     *dst = nullptr;
     const size_t bytes = std::max<size_t>(16, src.size() * sizeof(T));
-    if (hipMalloc(reinterpret_cast<void **>(dst), bytes) != hipSuccess) return MF_ERR_NOMEM;
+    if (mf::device_alloc(reinterpret_cast<void **>(dst), bytes) != MF_OK) return MF_ERR_NOMEM;
     if (!src.empty() &&
         hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice) != hipSuccess)
         return MF_ERR_HIP;

@@ -94,6 +94,8 @@ SIGNATURES = {
     "mf_graph_end": (_i, [_p, _p]),
     "mf_graph_launch": (_i, [_p, _p]),
     "mf_graph_destroy": (_i, [_p]),
+    "mf_workspace_bytes": (_i, [_p]),
+    "mf_workspace_release": (_i, []),
     "mf_plan_create": (_i, [_p, _i, _i, _i, _i, _p, _p, _p, _p, _p, _p]),
     "mf_plan_destroy": (_i, [_p]),
     "mf_plan_stats": (_i, [_p, _p]),

@@ -199,6 +199,20 @@ def synchronize():
     check(lib().mf_device_sync(), "mf_device_sync")
 
 
+def workspace_bytes():
+    """Bytes that the library's workspace pool on this GPU holds (mf_workspace_bytes)."""
+    _ensure()
+    out = ctypes.c_int64()
+    check(lib().mf_workspace_bytes(ctypes.byref(out)), "mf_workspace_bytes")
+    return out.value
+
+
+def workspace_release():
+    """Waits for the GPU and gives back what the pool keeps (mf_workspace_release)."""
+    _ensure()
+    check(lib().mf_workspace_release(), "mf_workspace_release")
+
+
 class Graph:
     """Work captured from a stream into an executable HIP graph, replayed as one
     submission (mf_graph_begin / mf_graph_end / mf_graph_launch)."""

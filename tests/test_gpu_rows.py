@@ -246,3 +246,21 @@ def test_large_lap_with_edges(mf, gpu):
                      coef=dm[4])
         got.append(values.numpy())
     same(got, "76^3")
+
+
+@pytest.mark.parametrize("edges", [False, True])
+def test_workspace_is_what_the_header_says(mf, gpu, edges):
+    """1.5 bytes an entry and color (of 32), with elemToEdge 4 an entry more, and what the pool
+    keeps is given back on request."""
+    print(f"[workspace] edges={edges}", flush=True)
+    coord, e2n, code, nnz = mf.generate_cube(40, 0.25, 3, 11)
+    m = mf.Mesh(coord, e2n, code, nnz, 0)
+    assert m.nbColors <= 32
+    dm = gpu.DeviceMesh(m, with_elem_to_edge=edges)
+    gpu.workspace_release()
+    assert gpu.workspace_bytes() == 0
+    dm.iterate_colored()
+    used = (48 + (4 if edges else 0)) * m.nnz
+    assert 0.8 * used < gpu.workspace_bytes() < used + (4 << 20)  # the pool's own rounding
+    gpu.workspace_release()
+    assert gpu.workspace_bytes() == 0
