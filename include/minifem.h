@@ -141,7 +141,8 @@ double mf_compute_double_norm(const double *tab, int64_t size);
  *     colorToElem in device memory, nbColors a host pointer), from the elements in
  *     dependency levels (an element is colored once every lower-index element sharing a
  *     node with it is), so the colors equal the sequential scan's. elemToNode 16-byte
- *     aligned (MF_ERR_ARG otherwise), as hipMalloc returns it. */
+ *     aligned (MF_ERR_ARG otherwise), as hipMalloc returns it; the other three take any
+ *     array of ints. */
 int mf_dev_create_nodeToElem(const int *elemToNode, int nbElem, int nbNodes, int *index,
                              int *value, void *stream);
 int mf_dev_create_nodeToNode(int *row, int *col, const int *n2eIndex, const int *n2eValue,
@@ -229,7 +230,8 @@ int mf_gather_probe(double *dst, const double *src, const int64_t *idx, int64_t 
  * there is no memory for it, it runs one launch per color instead. elemToEdge (device, 16
  * per element) gives the scatter positions; NULL selects the reference's default row search
  * (src/assembly.cc:415-421). colorToElem is a HOST array of nbColors+1 offsets (the
- * reference's global). Device: coord, values, row, col, elemToNode, elemToEdge. */
+ * reference's global). Device: coord, values, row, col, elemToNode (16-byte aligned, as
+ * hipMalloc returns it), elemToEdge. */
 int mf_assembly(const double *coord, double *values, const int *row, const int *col,
                 const int *elemToNode, const int *elemToEdge, int nbElem, int nbEdges,
                 int operatorDim, int operatorID, const int *colorToElem, int nbColors,

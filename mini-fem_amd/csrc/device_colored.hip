@@ -396,7 +396,7 @@ __global__ void __launch_bounds__(64)
                             kl[h] = 1.0;
                             if constexpr (ELA) kc[h] = mf::ela_coef(coef, el);
                             else if (coef) kl[h] = coef[el];
-                            if (EDGES) ids[h] = reinterpret_cast<const int4 *>(e2e)[(int64_t)el * 4 + jj[h]];
+                            if (EDGES) ids[h] = mf::load_four(e2e + ((int64_t)el * 4 + jj[h]) * 4);
                         }
 #pragma unroll
                         for (int h = 0; h < H; h++) {
@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(kListThreads)
     if (!left) return;
     const int64_t stride = (int64_t)gridDim.x * kListThreads;
     for (int64_t t = (int64_t)blockIdx.x * kListThreads + threadIdx.x; t < (int64_t)nE * 4; t += stride) {
-        const int4 p = reinterpret_cast<const int4 *>(e2e)[t];
+        const int4 p = mf::load_four(e2e + t * 4);
         const int at[4] = {p.x, p.y, p.z, p.w};
         int nx[4];
 #pragma unroll

@@ -28,6 +28,14 @@ __device__ __forceinline__ void wave_sync()
 // Two doubles as one 16-byte access at any multiple of 8 bytes, as a CSR row's values lie.
 using Two = double __attribute__((ext_vector_type(2), aligned(8)));
 
+// Four ints as one 16-byte access at any multiple of 4 bytes, as a caller's integers may lie.
+using Four = int __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ int4 load_four(const int *p)
+{
+    const Four v = *reinterpret_cast<const Four *>(p);
+    return make_int4(v.x, v.y, v.z, v.w);
+}
+
 // The current device's own pool of stream-ordered memory, for the workspaces of calls
 // (device_runtime.hip); null when it cannot be made. hipFreeAsync makes it safe for several
 // streams and threads.

@@ -118,7 +118,7 @@ __device__ int row_columns(int i, const int *__restrict__ index, const int *__re
 // lists in memory took 1.2 ms for a 50^3 cube's lengths and 0.26 for its columns; these two
 // take 83 and 20 us.)
 __global__ void __launch_bounds__(256)
-k_row_len(const int *__restrict__ index, const int *__restrict__ value, const int4 *__restrict__ e2n,
+k_row_len(const int *__restrict__ index, const int *__restrict__ value, const int *__restrict__ e2n,
           int N, int *__restrict__ len, uint8_t *__restrict__ flags)
 {
     __shared__ int4 s_elem[16][kListElems + 1];  // rows start on different banks
@@ -127,7 +127,7 @@ k_row_len(const int *__restrict__ index, const int *__restrict__ value, const in
     if (i >= N) return;
     const int b = index[i], L = index[i + 1] - b;
     if (L > kListElems) {  // more than the lanes hold: one lane through the lists in memory
-        if (l == 0) len[i] = row_columns(i, index, value, reinterpret_cast<const int *>(e2n), nullptr, 0);
+        if (l == 0) len[i] = row_columns(i, index, value, e2n, nullptr, 0);
         return;
     }
     int4 own[kListOwn];
@@ -135,7 +135,7 @@ k_row_len(const int *__restrict__ index, const int *__restrict__ value, const in
 #pragma unroll
     for (int h = 0; h < kListOwn; h++) {
         const int j = l + 16 * h;
-        own[h] = j < L ? e2n[value[b + j]] : make_int4(0, 0, 0, 0);
+        own[h] = j < L ? mf::load_four(e2n + (int64_t)value[b + j] * 4) : make_int4(0, 0, 0, 0);
         if (j < L) s_elem[g][j] = own[h];
         const int4 v = own[h];
         fresh[h] = 1u | (v.y != v.x) << 1 | (v.z != v.x && v.z != v.y) << 2 |
@@ -169,7 +169,7 @@ k_row_len(const int *__restrict__ index, const int *__restrict__ value, const in
 }
 
 __global__ void __launch_bounds__(256)
-k_row_fill(const int *__restrict__ index, const int *__restrict__ value, const int4 *__restrict__ e2n,
+k_row_fill(const int *__restrict__ index, const int *__restrict__ value, const int *__restrict__ e2n,
            const int *__restrict__ row, int N, const uint8_t *__restrict__ flags, int *__restrict__ col)
 {
     const int l = threadIdx.x & 15;
@@ -178,7 +178,7 @@ k_row_fill(const int *__restrict__ index, const int *__restrict__ value, const i
     const int b = index[i], L = index[i + 1] - b;
     if (L > kListElems) {
         if (l == 0)
-            row_columns(i, index, value, reinterpret_cast<const int *>(e2n), col + row[i], row[i + 1] - row[i]);
+            row_columns(i, index, value, e2n, col + row[i], row[i + 1] - row[i]);
         return;
     }
     int at = row[i];
@@ -194,7 +194,7 @@ k_row_fill(const int *__restrict__ index, const int *__restrict__ value, const i
         }
         int p = at + scan - n;
         if (f) {
-            const int4 q = e2n[value[b + j]];
+            const int4 q = mf::load_four(e2n + (int64_t)value[b + j] * 4);
             const int v[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
             for (int k = 0; k < 4; k++)
@@ -208,11 +208,11 @@ k_row_fill(const int *__restrict__ index, const int *__restrict__ value, const i
 // vertex pairs, row-major. A lane looks through one row for the four columns of an element,
 // four entries at a time.
 __global__ void k_elem_to_edge(const int *__restrict__ row, const int *__restrict__ col,
-                               const int4 *__restrict__ e2n, int nE, int4 *__restrict__ e2e)
+                               const int *__restrict__ e2n, int nE, int *__restrict__ e2e)
 {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= (int64_t)nE * 4) return;
-    const int4 v = e2n[t >> 2];
+    const int4 v = mf::load_four(e2n + (t >> 2) * 4);
     const int i = (int)(t & 3), a = (i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w) - 1;
     int4 p = make_int4(-1, -1, -1, -1);
     int left = 4;
@@ -229,7 +229,7 @@ __global__ void k_elem_to_edge(const int *__restrict__ row, const int *__restric
             if (p.w < 0 && c[u] == v.w) { p.w = q; left--; }
         }
     }
-    e2e[t] = p;
+    *reinterpret_cast<mf::Four *>(e2e + t * 4) = mf::Four{p.x, p.y, p.z, p.w};
 }
 
 inline dim3 grid_for(int64_t n, int bt) { return dim3((unsigned)((n + bt - 1) / bt)); }
@@ -776,11 +776,10 @@ extern "C" int mf_dev_create_nodeToNode(int *row, int *col, const int *n2eIndex,
     int *len = ws.cut<int>((size_t)N + 1);
     uint8_t *flags = ws.cut<uint8_t>((size_t)std::max(inc, 0) + 1);
     void *tmp = ws.cut<unsigned char>(scan_bytes + 1);
-    const int4 *e2n = reinterpret_cast<const int4 *>(elemToNode);
     if (hipMemsetAsync(len + N, 0, sizeof(int), s) != hipSuccess) return MF_ERR_HIP;
     if (N > 0)
-        hipLaunchKernelGGL(k_row_len, grid_for(N, 16), dim3(256), 0, s, n2eIndex, n2eValue, e2n, N, len,
-                           flags);
+        hipLaunchKernelGGL(k_row_len, grid_for(N, 16), dim3(256), 0, s, n2eIndex, n2eValue, elemToNode, N,
+                           len, flags);
     if (hipGetLastError() != hipSuccess ||
         hipcub::DeviceScan::ExclusiveSum(tmp, scan_bytes, len, row, N + 1, s) != hipSuccess ||
         hipMemcpyAsync(&nnz, row + N, sizeof(int), hipMemcpyDeviceToHost, s) != hipSuccess ||
@@ -789,8 +788,8 @@ extern "C" int mf_dev_create_nodeToNode(int *row, int *col, const int *n2eIndex,
     if (nnz > nbEdges) return MF_ERR_NNZ;  // the pattern does not fit col[]
     if (N > 0 && nnz > 0) {
         if (!col) return MF_ERR_ARG;
-        hipLaunchKernelGGL(k_row_fill, grid_for(N, 16), dim3(256), 0, s, n2eIndex, n2eValue, e2n, row, N,
-                           flags, col);
+        hipLaunchKernelGGL(k_row_fill, grid_for(N, 16), dim3(256), 0, s, n2eIndex, n2eValue, elemToNode, row,
+                           N, flags, col);
         if (hipGetLastError() != hipSuccess) return MF_ERR_HIP;
     }
     return hipStreamSynchronize(s) == hipSuccess ? nnz : MF_ERR_HIP;
@@ -804,8 +803,7 @@ extern "C" int mf_dev_create_elemToEdge(const int *row, const int *col, const in
     if (nbElem == 0) return MF_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     hipLaunchKernelGGL(k_elem_to_edge, grid_for((int64_t)nbElem * 4, 256), dim3(256), 0, s, row, col,
-                       reinterpret_cast<const int4 *>(elemToNode), nbElem,
-                       reinterpret_cast<int4 *>(elemToEdge));
+                       elemToNode, nbElem, elemToEdge);
     if (hipGetLastError() != hipSuccess) return MF_ERR_HIP;
     return hipStreamSynchronize(s) == hipSuccess ? MF_OK : MF_ERR_HIP;
 }

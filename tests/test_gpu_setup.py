@@ -172,3 +172,42 @@ def test_chains_and_rows_equal_host(mf, gpu, what):
     assert np.array_equal(d[2].numpy(), row)
     assert np.array_equal(d[3].numpy()[:d[5]], col[:d[5]])
     assert np.array_equal(d[4].numpy(), mf.create_elemToEdge(row, col, e2n))
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_setup_of_arrays_at_any_place(mf, gpu, off):
+    """nodeToElem, nodeToNode and elemToEdge read and write their arrays 16 bytes at a time,
+    and mf_assembly its elemToEdge: arrays that start at any int, in a larger buffer."""
+    print(f"[any place] off={off}", flush=True)
+    mesh = mf.Mesh.cube(9, 0.25, 3, 1)
+    n, nE, nnz = mesh.nbNodes, mesh.nbElem, mesh.nnz
+
+    def at(size, data=None):
+        room = gpu.DeviceArray.from_numpy(np.full(size + 8, -7, np.int32))
+        view = gpu.DeviceView(room.ptr + 4 * off, size, np.int32, owner=room)
+        if data is not None:
+            mf.check(mf.lib().mf_memcpy_h2d(view.ptr, data.ctypes.data, 4 * size, None), "h2d")
+        return view
+
+    def value_of(view, size):
+        whole = view._owner.numpy()
+        assert np.all(whole[:off] == -7) and np.all(whole[off + size:] == -7)
+        return whole[off:off + size]
+
+    e2n = at(4 * nE, mesh.elemToNode)
+    index, value, row, col, e2e = at(n + 1), at(4 * nE), at(n + 1), at(nnz), at(16 * nE)
+    lib = mf.lib()
+    mf.check(lib.mf_dev_create_nodeToElem(e2n.ptr, nE, n, index.ptr, value.ptr, None), "nodeToElem")
+    got = mf.check(lib.mf_dev_create_nodeToNode(row.ptr, col.ptr, index.ptr, value.ptr, e2n.ptr, n, nnz,
+                                                None), "nodeToNode")
+    mf.check(lib.mf_dev_create_elemToEdge(row.ptr, col.ptr, e2n.ptr, e2e.ptr, nE, None), "elemToEdge")
+    want = mf.create_elemToEdge(mesh.row, mesh.col, mesh.elemToNode)
+    assert got == nnz and np.array_equal(value_of(row, n + 1), mesh.row)
+    assert np.array_equal(value_of(col, nnz), mesh.col)
+    assert np.array_equal(value_of(e2e, 16 * nE), want)
+    dm, values = gpu.DeviceMesh(mesh), []
+    for edges in (gpu.DeviceArray.from_numpy(want), e2e):
+        gpu.assembly(dm.coord, dm.values, row, col, dm.elemToNode, edges, nE, nnz, 9, 1,
+                     mesh.colorToElem)
+        values.append(dm.values.numpy())
+    assert np.array_equal(values[0], values[1])
