@@ -166,10 +166,10 @@ __global__ void __launch_bounds__(kBT)
 // The ela product with the value stream staged through LDS: a wave's four row groups own
 // four consecutive rows, whose blocks are one contiguous segment of values; the wave
 // reads it in chunks of kChunk blocks with consecutive lanes on consecutive 16-byte
-// pieces (the per-lane 72-byte blocks of k_spmv touch each line from several lanes and
-// several instructions), then every lane takes its blocks from LDS in k_spmv's order, so
-// the sums, and q, are k_spmv's bit for bit. Only this wave reads its LDS region, and LDS
-// operations of one wave complete in order, so no workgroup barrier is needed.
+// pieces (a lane that reads its own 72-byte block touches each line with several lanes and
+// several instructions), then every lane takes its row's blocks from LDS in turn, every
+// 16th, as the lanes of the lap product take entries. Only this wave reads its LDS region, and
+// LDS operations of one wave complete in order, so no workgroup barrier is needed.
 constexpr int kChunk = 64;
 __global__ void __launch_bounds__(kBT)
     k_spmv_ela_staged(const int *__restrict__ row, const int *__restrict__ col,

@@ -235,7 +235,7 @@ __device__ __forceinline__ int seek(const XcdWalk<Jobs> &W, Cursor &c, int p)
 }
 
 // LDS layout of tile hh as operator ELA runs it. FRONT_ELA: the fixed front part holds
-// ela coefficients (16 bytes per element); a launch that mixes operators sizes it so for
+// ela coefficients (mf::front_coef_bytes); a launch that mixes operators sizes it so for
 // every tile, since the loaders fill the next tile's front while the current one runs.
 template <bool ELA, int PREC, bool FRONT_ELA>
 __device__ __forceinline__ mf::TileLds tile_layout(const mf::TileHdr &hh, int f_node, int f_elem)

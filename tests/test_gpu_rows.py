@@ -72,6 +72,18 @@ def test_rows_of_many_elements(mf, gpu, op, n):
             same(both(mf, gpu, m, e2e, precision=precision), n)
 
 
+@pytest.mark.parametrize("op", [0, 1])
+@pytest.mark.parametrize("n", [23, 24, 25, 47, 48, 49, 72, 73, 96, 120, 121, 128])
+def test_rows_at_the_chunks_edges(mf, gpu, op, n):
+    """A row's elements are staged 24 at a time: one full chunk to five, one element more and
+    one less, and the most colors there are."""
+    print(f"[rows chunks] op={op} n={n}", flush=True)
+    m = fan(n, op, mf)
+    for e2e in (None, mf.create_elemToEdge(m.row, m.col, m.elemToNode)):
+        for precision in (0, 1):
+            same(both(mf, gpu, m, e2e, precision=precision), n)
+
+
 @pytest.mark.parametrize("op,n", [(0, 6), (1, 6), (0, 13), (1, 13)])
 def test_rows_odd_patterns(mf, gpu, op, n):
     coord, e2n, code, nnz = mf.generate_cube(n, 0.25, 3, 11)
