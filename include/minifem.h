@@ -466,7 +466,8 @@ typedef struct mf_server_stats {
     double makespan_s;     /* first arrival to last completion */
 } mf_server_stats;
 
-/* arena: device memory of arena_bytes that the server carves for request inputs and
+/* arena: device memory of arena_bytes (the library's workspace pool, mf_workspace_bytes, is
+ * besides) that the server carves for request inputs and
  * outputs (no allocation while serving); slots: streams (1..16); max_group:
  * 1..MF_MAX_PLAN_JOBS; max_bypass >= 0. */
 int mf_server_create(mf_server **server, void *arena, int64_t arena_bytes, int slots,

@@ -667,8 +667,8 @@ __global__ void __launch_bounds__(kSumThreads)
 // kLeftGrid-th row, looks through all elements of a color for vertices of its own, and adds their
 // blocks once the color is listed, 16 lanes an element. Lanes of one element that share an entry
 // (a vertex stands twice in it) add in order, on one lane. Reading the elements kLeftGrid times is
-// what it costs: ela 40^3 with one element that repeats a vertex 1,045 us, one launch per color
-// 519, all colors in one workgroup 61,700.
+// what it costs; a workgroup a CU is the best (ela 40^3 with one element that repeats a vertex 1,045
+// us, 128 of them 1,708, 512 1,272; one launch per color 519, all colors in one workgroup 61,700).
 constexpr int kLeftGrid = 256, kLeftThreads = 1024;
 
 template <int OP, int PREC>
