@@ -713,7 +713,7 @@ __global__ void __launch_bounds__(kLeftThreads)
                 const int v[4] = {q.x, q.y, q.z, q.w};
                 const int nj = j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
                 const int nk = k == 0 ? v[0] : k == 1 ? v[1] : k == 2 ? v[2] : v[3];
-                int p = own(nj) ? elem_position(row, col, nullptr, e, nj, nk, l) : -1;
+                int p = nj > 0 && own(nj) ? elem_position(row, col, nullptr, e, nj, nk, l) : -1;
                 if (p >= nnz) p = -1;
                 bool twice = false;
 #pragma unroll
